@@ -100,13 +100,15 @@ __device__ void block_exclusive_scan_n(const int (&v)[NV], int (&excl)[NV], int 
   for (int k = 0; k < NV; ++k) excl[k] = wr < 0 ? 0 : wr < nv ? x[k] - v[k] + pre[k] : total[k];
 }
 
-// Token blocks (32 slots) of the tallest MFMA tile: the tile list is ordered
-// by height class, tallest first.
+// Token blocks of the tallest tile (MFMA tiles: 32 slots a block; exact-weight
+// tiles: 16): the tile list is ordered by height class, tallest first.
 constexpr int kTileClasses = kMfmaTileMMax / 32;
+static_assert(kXTileM / 16 <= kTileClasses, "height classes of the exact-weight tiles");
+__device__ __forceinline__ int block_shift(const AlignLaunch& a) { return a.xtiles ? 4 : 5; }
 
 // Work lists of the fused call.  An expert with more than gemv_max_tokens
 // pairs gets ceil(count / tile_m) MFMA tiles of near-equal size (multiples of
-// 32 slots but the last); the tiles are listed by height class, tallest
+// 32 slots, exact-weight tiles of 16, but the last); the tiles are listed by height class, tallest
 // first (experts ascending within a class), so that the MFMA launch starts
 // its longest tiles first.  Every other routed expert's single sorted block
 // goes to the GEMV list.  Thread tid owns experts e0 .. e0 + ipt - 1.
@@ -130,10 +132,11 @@ __device__ __forceinline__ int div_small(int n, int d) {
   return q;
 }
 
-// Tile height and count of an expert with c > gemv_max_tokens pairs.
-__device__ __forceinline__ void tile_split(int c, int tile_m, int& per, int& n_t) {
+// Tile height and count of an expert with c > gemv_max_tokens pairs, in
+// blocks of 1 << bs slots.
+__device__ __forceinline__ void tile_split(int c, int tile_m, int bs, int& per, int& n_t) {
   const int n_ch = div_small(c + tile_m - 1, tile_m);
-  per = (div_small(c + n_ch - 1, n_ch) + 31) & ~31;  // <= tile_m
+  per = (div_small(c + n_ch - 1, n_ch) + (1 << bs) - 1) >> bs << bs;  // <= tile_m
   n_t = div_small(c + per - 1, per);
 }
 
@@ -145,9 +148,9 @@ __device__ __forceinline__ int round_up_block(int c, int B) {
 __device__ void scan_inputs(const AlignLaunch& a, const int32_t* tot, int e0, int ipt,
                             int (&v)[kScanSlots]) {
   constexpr int NC = kTileClasses;
-  const int E = a.num_experts, B = a.block, thr = a.gemv_max_tokens;
+  const int E = a.num_experts, B = a.block, thr = a.gemv_max_tokens, bs = block_shift(a);
   // class of a tile of n slots: NC - (token blocks)
-  auto cls = [](int n) { return NC - ((n + 31) >> 5); };
+  auto cls = [bs](int n) { return NC - ((n + (1 << bs) - 1) >> bs); };
 #pragma unroll
   for (int k = 0; k < kScanSlots; ++k) v[k] = 0;
   for (int i = 0; i < ipt; ++i) {
@@ -155,10 +158,10 @@ __device__ void scan_inputs(const AlignLaunch& a, const int32_t* tot, int e0, in
     if (e >= E) break;
     const int c = tot[e];
     v[NC + 1] += round_up_block(c, B);
-    if (!a.tiles) continue;
+    if (!a.n_tiles) continue;
     if (c > thr) {
       int per, n_t;
-      tile_split(c, a.tile_m, per, n_t);
+      tile_split(c, a.tile_m, bs, per, n_t);
       const int kf = cls(per), kl = cls(c - (n_t - 1) * per);
 #pragma unroll
       for (int k = 0; k < NC; ++k) v[k] += (k == kf ? n_t - 1 : 0) + (k == kl ? 1 : 0);
@@ -172,8 +175,8 @@ __device__ void write_work_lists(const AlignLaunch& a, const int32_t* tot, const
                                  int e0, int ipt, const int (&excl)[kScanSlots],
                                  const int (&total)[kScanSlots], bool scalars) {
   constexpr int NC = kTileClasses;
-  const int E = a.num_experts, B = a.block, thr = a.gemv_max_tokens;
-  auto cls = [](int n) { return NC - ((n + 31) >> 5); };
+  const int E = a.num_experts, B = a.block, thr = a.gemv_max_tokens, bs = block_shift(a);
+  auto cls = [bs](int n) { return NC - ((n + (1 << bs) - 1) >> bs); };
   int pos[NC + 1];
   int n_tiles = 0;
 #pragma unroll
@@ -188,7 +191,7 @@ __device__ void write_work_lists(const AlignLaunch& a, const int32_t* tot, const
     const int c = tot[e];
     if (c > thr) {
       int per, n_t;
-      tile_split(c, a.tile_m, per, n_t);
+      tile_split(c, a.tile_m, bs, per, n_t);
       for (int s0 = 0; s0 < c; s0 += per) {
         const int n = min(per, c - s0);
         const int k = cls(n);
@@ -196,7 +199,10 @@ __device__ void write_work_lists(const AlignLaunch& a, const int32_t* tot, const
 #pragma unroll
         for (int j = 0; j < NC; ++j)
           if (j == k) p = pos[j]++;
-        a.tiles[p] = make_int4(e, off[e] + s0, n, 0);
+        if (a.xtiles)
+          a.xtiles[p] = ((off[e] + s0) >> 4) | (((n + 15) >> 4) << 28);
+        else
+          a.tiles[p] = make_int4(e, off[e] + s0, n, 0);
       }
     } else if (c > 0) {
       a.gemv_blocks[pos[NC]++] = div_small(off[e], B);
@@ -204,7 +210,7 @@ __device__ void write_work_lists(const AlignLaunch& a, const int32_t* tot, const
   }
   if (scalars) {
     a.n_tiles[0] = n_tiles;
-    a.n_gemv[0] = total[NC];
+    if (a.n_gemv) a.n_gemv[0] = total[NC];
   }
 }
 
@@ -371,7 +377,7 @@ __global__ __launch_bounds__(1024) void align_kernel(const AlignLaunch a) {
   // lists of the fused call, block experts and scalars, everyone's share of
   // the padding -- while the placement writes the other sorted positions
   if (own >= 0 && own < n_own) {
-    if (a.tiles) write_work_lists(a, tot, off, e0, ipt, sx, st, own == 0);
+    if (a.n_tiles) write_work_lists(a, tot, off, e0, ipt, sx, st, own == 0);
     write_block_experts(a, off, e0, ipt);
     if (a.offsets)
       for (int e = own; e <= E; e += n_own) a.offsets[e] = off[e];
@@ -567,7 +573,7 @@ __global__ __launch_bounds__(kChunk) void align_place_kernel(const AlignLaunch a
   if (g != 0) return;
 
   // 6. workgroup 0: work lists, sentinels, block experts, scalars
-  if (a.tiles) write_work_lists(a, tot, off, e0, ipt, sx, st, tid == 0);
+  if (a.n_tiles) write_work_lists(a, tot, off, e0, ipt, sx, st, tid == 0);
   write_block_experts(a, off, e0, ipt);
   write_padding(a, tot, off, total, tid, kChunk);
   if (a.offsets)

@@ -57,8 +57,10 @@ struct Layout {
   bool chunked;       // the sort runs over many workgroups (chunk counts at off_chunks)
   size_t off_chunks;
   bool route;         // GEMV kernels route themselves; no align kernel
+  bool xtile;         // every expert on the exact-weight MFMA tiles
+  int xtile_m;        // their height (slots)
   int tile_m;         // MFMA tile height (slots)
-  int64_t max_tiles;  // bound of the MFMA tile list
+  int64_t max_tiles;  // bound of the MFMA (or exact-weight) tile list
   int64_t max_gemv;   // bound of the GEMV block list / GEMV work items
   int64_t max_items;  // self-routed work items: one per (token, slot) pair
   bool token;         // one token: w2 and the combine in one launch
@@ -67,7 +69,7 @@ struct Layout {
   int tc;
   int upw;
   int lpr;
-  int row_tiles_w13;  // 256-row weight blocks per MFMA work item
+  int row_tiles_w13;  // 256-row weight blocks per MFMA (or exact-weight) work item
   int row_tiles_w2;
 };
 
@@ -141,6 +143,25 @@ int small_row_tiles(int64_t n_blocks, int64_t rows) {
   for (int r = 1; r <= n_blocks && r * (int64_t)kMfmaTileN <= rows; ++r)
     if (n_blocks % r == 0) best = r;
   return best;
+}
+// Height of the exact-weight tiles (xtile.hip) by average pairs per expert:
+// 32 slots below 24 pairs (the kernel of short tiles holds a second set of
+// activation rows and fragments in registers: E=256, K=3072, N=1024, 10 pairs
+// per expert, w13 192 us against 224), else 64 (80 pairs per expert at N=128:
+// 80 us against 90 with 48-slot tiles), or 48 for groups of 128, whose
+// fragments of a whole group do not fit the registers of taller tiles.
+constexpr int64_t kXTile32MaxPairs = 24;
+constexpr int kXTile128 = 48;
+// Row tiles (`rows` outputs each) one workgroup of the exact-weight tiles runs
+// in turn: about 16 steps of 128 elements, so that short reductions do not
+// pay a workgroup's first loads for each row tile, with six workgroups per CU
+// left for balance.
+int xtile_row_tiles(int64_t n_out, int64_t kdim, int64_t rows, int64_t max_tiles) {
+  const int64_t n_rt = (n_out + rows - 1) / rows;
+  const int64_t steps = (kdim + 127) / 128;
+  const int64_t want = std::max<int64_t>(1, 16 / steps);
+  const int64_t fill = std::max<int64_t>(1, max_tiles * n_rt / (6 * kCUs));
+  return (int)std::min<int64_t>(n_rt, std::min(want, fill));
 }
 // Average (token, slot) pairs per expert from which the built-in split sends
 // every expert to the MFMA kernels (gemv_max_tokens 0, no GEMV launches).
@@ -219,7 +240,18 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
   // launches that would look for one cost more than an MFMA tile for it, so
   // every expert goes to the MFMA kernels and the GEMV launches are skipped.
   if (L->mfma && T.auto_split && (int64_t)n_tok >= kAllMfmaMinPairs * E) L->gemv_max_tokens = 0;
-  L->gemv = !L->mfma || L->gemv_max_tokens > 0;
+  // Small batches: the GEMV kernels route themselves from topk_ids (work
+  // item = one routed expert), so the align kernel is not run.
+  L->route = !L->mfma && M >= 1 && M <= T.gemv_only_max_m &&
+             gemv_route_fits((int)n_tok, (int)E, (int)K, (int)N);
+  // Every other call that keeps all experts on exact weights (K or N no
+  // multiple of 256, scales that are not 16-byte aligned, or by the tuning):
+  // MFMA tiles of exact weights, any K and N the library takes.  The GEMV's
+  // passes of four rows, which ran them before, cost a pass over the weights
+  // per four pairs: E=256, K=3072, N=128, 80 pairs per expert 1,272 -> 207 us
+  // per call; E=64, K=2048, N=1408, group 128, 73 pairs 1,351 -> 203 us.
+  L->xtile = !L->mfma && !L->route;
+  L->gemv = L->mfma ? L->gemv_max_tokens > 0 : L->route;
   L->tc = T.tc;
   L->upw = T.upw;
   L->lpr = T.lpr;
@@ -241,12 +273,15 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
     L->row_tiles_w2 = pick_row_tiles(K / kMfmaTileN, N / 64, n_tok, E, kItemWorkW2);
   }
   L->max_tiles = L->mfma ? (int64_t)n_tok / L->tile_m + heavy : 0;
-  L->max_gemv = L->mfma ? std::min<int64_t>(std::min<int64_t>(E, (int64_t)n_tok), L->nb)
-                        : std::min<int64_t>((int64_t)n_tok, L->nb);
-  // Small batches: the GEMV kernels route themselves from topk_ids (work
-  // item = one routed expert), so the align kernel is not run.
-  L->route = !L->mfma && M >= 1 && M <= T.gemv_only_max_m &&
-             gemv_route_fits((int)n_tok, (int)E, (int)K, (int)N);
+  if (L->xtile) {
+    L->xtile_m = (int64_t)n_tok < kXTile32MaxPairs * E ? 32 : group == 128 ? kXTile128 : kXTileM;
+    // (never more than the sorted 16-slot blocks that hold a pair)
+    L->max_tiles = std::min<int64_t>((int64_t)n_tok / L->xtile_m + std::min<int64_t>(E, n_tok),
+                                     std::min<int64_t>(n_tok, L->nb));
+    L->row_tiles_w13 = xtile_row_tiles(N, K, 128, L->max_tiles);
+    L->row_tiles_w2 = xtile_row_tiles(K, N, 256, L->max_tiles);
+  }
+  L->max_gemv = L->mfma ? std::min<int64_t>(std::min<int64_t>(E, (int64_t)n_tok), L->nb) : 0;
   L->max_items = L->route ? (int64_t)n_tok : 0;
   L->token = L->route && M <= T.w2_fused_max_m && w2_token_fits((int)topk, (int)K, (int)N);
   L->partial_bf16 = M > kFp32PartialMaxM;
@@ -261,7 +296,8 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
   put(W4A16_WS_OFFSETS, (size_t)(E + 1) * sizeof(int32_t));
   put(W4A16_WS_INTER, n_tok * (size_t)N * sizeof(uint16_t));
   put(W4A16_WS_PARTIAL, n_tok * (size_t)K * (L->partial_bf16 ? sizeof(uint16_t) : sizeof(float)));
-  put(W4A16_WS_TILES, (size_t)std::max<int64_t>(L->max_tiles, 1) * 4 * sizeof(int32_t));
+  put(W4A16_WS_TILES, (size_t)std::max<int64_t>(L->max_tiles, 1) *
+                          (L->xtile ? sizeof(int32_t) : sizeof(int4)));
   put(W4A16_WS_GEMV_BLOCKS, (size_t)std::max<int64_t>(L->max_gemv, 1) * sizeof(int32_t));
   // Internal (not one of the public fields): the chunk counts of the
   // many-workgroup sort of large batches.
@@ -358,7 +394,7 @@ Work work_of(const Layout& L, void* ws_base) {
 // The GEMV launch of GEMM `mode` (0: w13, 1: w2).
 GemvLaunch gemv_args(const FusedArgs& a, const Layout& L, const Work& w, int mode) {
   GemvLaunch g{};
-  g.block_list = L.mfma ? w.gemv_blocks : nullptr;
+  g.block_list = L.route ? nullptr : w.gemv_blocks;
   g.sorted = w.sorted;
   g.expert_ids = w.eids;
   g.header = w.header;
@@ -440,6 +476,42 @@ MfmaLaunch mfma_args(const FusedArgs& a, const Layout& L, const Work& w, int mod
   return m;
 }
 
+// The exact-weight tile launch of GEMM `mode`.
+XtileLaunch xtile_args(const FusedArgs& a, const Layout& L, const Work& w, int mode) {
+  XtileLaunch x{};
+  x.sorted = w.sorted;
+  x.expert_ids = w.eids;
+  x.tiles = reinterpret_cast<const int32_t*>(w.tiles);
+  x.header = w.header;
+  x.n_tok = (int32_t)(a.M * a.topk);
+  x.topk = (int32_t)a.topk;
+  x.group = (int32_t)a.group;
+  x.max_tiles = (int32_t)L.max_tiles;
+  x.tile_m = L.xtile_m;
+  if (mode == 0) {
+    x.act = static_cast<const uint16_t*>(a.hidden);
+    x.ld_act = a.ld_hidden;
+    x.w = static_cast<const uint32_t*>(a.w13);
+    x.s = static_cast<const uint16_t*>(a.s13);
+    x.out = w.inter;
+    x.n_out = (int32_t)a.N;
+    x.kdim = (int32_t)a.K;
+    x.row_tiles = L.row_tiles_w13;
+  } else {
+    x.act = w.inter;
+    x.ld_act = a.N;
+    x.w = static_cast<const uint32_t*>(a.w2);
+    x.s = static_cast<const uint16_t*>(a.s2);
+    x.topk_w = a.topk_w;
+    x.out = w.partial;
+    x.partial_bf16 = L.partial_bf16;
+    x.n_out = (int32_t)a.K;
+    x.kdim = (int32_t)a.N;
+    x.row_tiles = L.row_tiles_w2;
+  }
+  return x;
+}
+
 // Whether GEMM `mode` of the split dispatch (GEMV and MFMA work items both)
 // runs as one mixed launch.
 bool mixed_launch(const FusedArgs& a, const Layout& L, const Work& w, int mode) {
@@ -471,7 +543,11 @@ int run_fused(const FusedArgs& a, const Layout& L, hipStream_t stream, hipEvent_
   al.offsets = w.offsets;
   al.dropped = w.header + 1;
   al.chunk_scratch = w.chunks;
-  if (L.mfma) {
+  if (L.xtile) {
+    al.xtiles = reinterpret_cast<int32_t*>(w.tiles);
+    al.n_tiles = w.header + 2;
+    al.tile_m = L.xtile_m;
+  } else if (L.mfma) {
     al.tiles = w.tiles;
     al.n_tiles = w.header + 2;
     al.gemv_blocks = w.gemv_blocks;
@@ -487,7 +563,9 @@ int run_fused(const FusedArgs& a, const Layout& L, hipStream_t stream, hipEvent_
   if (want(1)) {
     const GemvLaunch g = gemv_args(a, L, w, 0);
     const MfmaLaunch m = mfma_args(a, L, w, 0);
-    if (mixed_launch(a, L, w, 0)) {
+    if (L.xtile) {
+      if (launch_w13_xtile(xtile_args(a, L, w, 0), stream) != hipSuccess) return W4A16_ERR_HIP;
+    } else if (mixed_launch(a, L, w, 0)) {
       if (launch_w13_mixed(m, g, stream) != hipSuccess) return W4A16_ERR_HIP;
     } else {
       if (L.gemv && launch_w13_gemv(g, stream) != hipSuccess) return W4A16_ERR_HIP;
@@ -504,6 +582,8 @@ int run_fused(const FusedArgs& a, const Layout& L, hipStream_t stream, hipEvent_
     if (L.token) {
       if (launch_w2_token(g, static_cast<uint16_t*>(a.out), a.ld_out, stream) != hipSuccess)
         return W4A16_ERR_HIP;
+    } else if (L.xtile) {
+      if (launch_w2_xtile(xtile_args(a, L, w, 1), stream) != hipSuccess) return W4A16_ERR_HIP;
     } else if (mixed_launch(a, L, w, 1)) {
       if (launch_w2_mixed(m, g, stream) != hipSuccess) return W4A16_ERR_HIP;
     } else {
@@ -712,7 +792,7 @@ int w4a16_moe_stage_launches(int64_t M, int64_t topk, int64_t num_experts, int64
                     group_size, const_cast<void*>(p), K, const_cast<void*>(p), L.total, tuning};
   const Work w = work_of(L, const_cast<void*>(p));
   auto gemm = [&](int mode) {
-    return mixed_launch(a, L, w, mode) ? 1 : (L.gemv ? 1 : 0) + (L.mfma ? 1 : 0);
+    return L.xtile || mixed_launch(a, L, w, mode) ? 1 : (L.gemv ? 1 : 0) + (L.mfma ? 1 : 0);
   };
   launches[0] = L.route ? 0 : (L.chunked ? 2 : 1);
   launches[1] = gemm(0);

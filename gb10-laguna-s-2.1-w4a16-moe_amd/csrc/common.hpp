@@ -124,6 +124,7 @@ struct AlignLaunch {
   // their single sorted block on the GEMV path.
   // Requires gemv_max_tokens < block.
   int4* tiles;           // [max tiles] (expert, first slot, count, 0)
+  int32_t* xtiles;       // exact-weight tiles instead: first slot / 16 | blocks of 16 << 28
   int32_t* n_tiles;      // [1]
   int32_t* gemv_blocks;  // [max blocks] block indices, ascending
   int32_t* n_gemv;       // [1]
@@ -161,8 +162,8 @@ struct GemvLaunch {
   int32_t group;
   int32_t max_blocks;      // upper bound of active blocks
   int32_t num_experts;
-  const int32_t* block_list;  // null: work item b is block b; else blocks
-                              // block_list[0 .. header[3])
+  const int32_t* block_list;  // work item b is block block_list[b], b < header[3]
+                              // (not read by self-routing calls)
   uint32_t nib_mask;          // set by the launcher (see gemv.hip)
   uint32_t nib_magic;
   // Self-routing (small batches, the align kernel is not run): when `ids`
@@ -214,6 +215,35 @@ struct MfmaLaunch {
 };
 hipError_t launch_w13_mfma(const MfmaLaunch& a, hipStream_t stream);
 hipError_t launch_w2_mfma(const MfmaLaunch& a, hipStream_t stream);
+
+// Exact-weight tiles (xtile.hip): an expert's pairs are cut into tiles of at
+// most kXTileM slots.
+constexpr int kXTileM = 64;
+struct XtileLaunch {
+  const uint16_t* act;     // bf16 activation rows (x for w13, inter for w2)
+  int64_t ld_act;
+  const uint32_t* w;       // packed weights [E, rows_total, kdim/8]
+  const uint16_t* s;       // bf16 scales   [E, rows_total, kdim/G]
+  const int32_t* sorted;
+  const int32_t* expert_ids;
+  const int32_t* tiles;    // first slot / 16 | blocks of 16 slots << 28
+  const int32_t* header;   // [2] = number of tiles
+  const float* topk_w;     // w2 only
+  void* out;               // w13: bf16 inter [n_tok, n_out]; w2: partial [n_tok, n_out]
+  int32_t partial_bf16;    // w2: partial rows are bf16 (else fp32)
+  int32_t n_tok;
+  int32_t topk;
+  int32_t n_out;           // N for w13 (2N weight rows), K for w2
+  int32_t kdim;
+  int32_t group;
+  int32_t max_tiles;
+  int32_t tile_m;          // slots per tile, at most (<= kXTileM)
+  int32_t row_tiles;       // row tiles (256 weight rows) one workgroup runs in turn
+  uint32_t nib_mask;       // set by the launcher
+  uint32_t nib_magic;
+};
+hipError_t launch_w13_xtile(const XtileLaunch& a, hipStream_t stream);
+hipError_t launch_w2_xtile(const XtileLaunch& a, hipStream_t stream);
 
 // The split dispatch's GEMV and MFMA work items of one GEMM (mode 0: w13,
 // 1: w2) in one launch, when mixed_fits(mode, m, g): m and g are the two
