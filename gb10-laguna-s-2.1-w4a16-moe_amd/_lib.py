@@ -51,6 +51,8 @@ GEMV_ONLY_MAX_M = 24
 EXPORTED_SYMBOLS = (
     "w4a16_moe_align_sizes",
     "w4a16_moe_align_block_size",
+    "w4a16_moe_align_scratch_size",
+    "w4a16_moe_align_block_size_ws",
     "w4a16_moe_workspace_size",
     "w4a16_moe_workspace_layout",
     "w4a16_moe_fused_experts",
@@ -100,6 +102,11 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.w4a16_moe_align_block_size.restype = ctypes.c_int
     lib.w4a16_moe_align_block_size.argtypes = [
         _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp]
+    lib.w4a16_moe_align_scratch_size.restype = ctypes.c_int
+    lib.w4a16_moe_align_scratch_size.argtypes = [_i64, _i64, _i64, ctypes.POINTER(ctypes.c_size_t)]
+    lib.w4a16_moe_align_block_size_ws.restype = ctypes.c_int
+    lib.w4a16_moe_align_block_size_ws.argtypes = [
+        _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp]
     lib.w4a16_moe_workspace_size.restype = ctypes.c_int
     lib.w4a16_moe_workspace_size.argtypes = [
         _i64, _i64, _i64, _i64, _i64, _i64, ctypes.POINTER(ctypes.c_size_t)]
@@ -168,6 +175,12 @@ def align_sizes(M: int, topk: int, num_experts: int, block_size: int) -> tuple[i
                                      ctypes.byref(em), ctypes.byref(nb))
     check(st)
     return em.value, nb.value
+
+
+def align_scratch_size(M: int, topk: int, num_experts: int) -> int:
+    out = ctypes.c_size_t()
+    check(lib().w4a16_moe_align_scratch_size(M, topk, num_experts, ctypes.byref(out)))
+    return out.value
 
 
 def workspace_size(M: int, topk: int, E: int, N: int, K: int, group: int) -> int:

@@ -593,7 +593,7 @@ __global__ __launch_bounds__(kChunk) void align_place_kernel(const AlignLaunch a
 int align_chunks(int n_tok) { return (n_tok + kChunk - 1) / kChunk; }
 
 hipError_t launch_align(const AlignLaunch& a, hipStream_t stream) {
-  if (a.chunk_scratch && a.n_tok >= kAlignChunkedMinPairs && a.num_experts <= kAlignChunkedMaxE) {
+  if (a.chunk_scratch && align_is_chunked(a.n_tok, a.num_experts)) {
     const int n_chunks = align_chunks(a.n_tok);
     int32_t* ctot = a.chunk_scratch;
     int32_t* cdrop = a.chunk_scratch + (size_t)n_chunks * a.num_experts;

@@ -301,7 +301,7 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
   put(W4A16_WS_GEMV_BLOCKS, (size_t)std::max<int64_t>(L->max_gemv, 1) * sizeof(int32_t));
   // Internal (not one of the public fields): the chunk counts of the
   // many-workgroup sort of large batches.
-  L->chunked = !L->route && (int64_t)n_tok >= kAlignChunkedMinPairs && E <= kAlignChunkedMaxE;
+  L->chunked = !L->route && align_is_chunked((int64_t)n_tok, E);
   L->off_chunks = cur;
   if (L->chunked) cur = round_up(cur + align_chunk_scratch_ints((int)n_tok, (int)E) * 4, kWsAlign);
   L->total = cur;
@@ -679,15 +679,44 @@ int w4a16_moe_align_sizes(int64_t M, int64_t topk, int64_t num_experts,
                      max_num_m_blocks);
 }
 
+int w4a16_moe_align_scratch_size(int64_t M, int64_t topk, int64_t num_experts, size_t* bytes) {
+  if (!bytes) return W4A16_ERR_NULL_POINTER;
+  int64_t em = 0, nb = 0;
+  const int st = align_sizes(M, topk, num_experts, 1, &em, &nb);
+  if (st) return st;
+  *bytes = align_is_chunked(M * topk, num_experts)
+               ? align_chunk_scratch_ints((int)(M * topk), (int)num_experts) * sizeof(int32_t)
+               : 0;
+  return W4A16_OK;
+}
+
 int w4a16_moe_align_block_size(const int32_t* topk_ids, int64_t M, int64_t topk,
                                int64_t num_experts, int64_t block_size,
                                int32_t* sorted_token_ids, int32_t* expert_ids,
                                int32_t* num_tokens_post_padded,
                                int32_t* expert_offsets, int32_t* dropped,
                                void* stream) {
+  return w4a16_moe_align_block_size_ws(topk_ids, M, topk, num_experts, block_size,
+                                       sorted_token_ids, expert_ids, num_tokens_post_padded,
+                                       expert_offsets, dropped, nullptr, 0, stream);
+}
+
+int w4a16_moe_align_block_size_ws(const int32_t* topk_ids, int64_t M, int64_t topk,
+                                  int64_t num_experts, int64_t block_size,
+                                  int32_t* sorted_token_ids, int32_t* expert_ids,
+                                  int32_t* num_tokens_post_padded,
+                                  int32_t* expert_offsets, int32_t* dropped,
+                                  void* scratch, size_t scratch_bytes, void* stream) {
   int64_t em = 0, nb = 0;
-  const int st = align_sizes(M, topk, num_experts, block_size, &em, &nb);
+  int st = align_sizes(M, topk, num_experts, block_size, &em, &nb);
   if (st) return st;
+  if (scratch) {
+    size_t need = 0;
+    st = w4a16_moe_align_scratch_size(M, topk, num_experts, &need);
+    if (st) return st;
+    if (scratch_bytes < need) return W4A16_ERR_WORKSPACE_TOO_SMALL;
+    if (!aligned(scratch, 4)) return W4A16_ERR_MISALIGNED;
+  }
   // zero-length outputs (M = 0 with block 1) may be NULL
   if ((M > 0 && !topk_ids) || (em > 0 && !sorted_token_ids) || (nb > 0 && !expert_ids) ||
       !num_tokens_post_padded)
@@ -704,6 +733,7 @@ int w4a16_moe_align_block_size(const int32_t* topk_ids, int64_t M, int64_t topk,
   al.num_post = num_tokens_post_padded;
   al.offsets = expert_offsets;
   al.dropped = dropped;
+  if (align_is_chunked(M * topk, num_experts)) al.chunk_scratch = static_cast<int32_t*>(scratch);
   (void)hipGetLastError();
   return launch_align(al, static_cast<hipStream_t>(stream)) == hipSuccess ? W4A16_OK
                                                                          : W4A16_ERR_HIP;

@@ -137,6 +137,9 @@ struct AlignLaunch {
 };
 constexpr int kAlignChunkedMinPairs = 8192;
 constexpr int kAlignChunkedMaxE = 512;
+inline bool align_is_chunked(int64_t n_tok, int64_t num_experts) {
+  return n_tok >= kAlignChunkedMinPairs && num_experts <= kAlignChunkedMaxE;
+}
 int align_chunks(int n_tok);
 inline size_t align_chunk_scratch_ints(int n_tok, int num_experts) {
   return (size_t)align_chunks(n_tok) * (num_experts + 1);

@@ -168,18 +168,8 @@ def _ids_i32(topk_ids: torch.Tensor) -> torch.Tensor:
     return topk_ids.contiguous()
 
 
-def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: int):
-    """Sort token-slots by expert and pad each expert to a multiple of block_size.
-
-    Returns (sorted_token_ids int32[EM], expert_ids int32[EM/B],
-    num_tokens_post_padded int32[1]) with EM = round_up(M*topk + E*(B-1), B),
-    bit-identical to kernels/w4a16_moe.py:187-290.  One HIP launch on the
-    current stream, no host synchronisation.
-    """
-    if not topk_ids.is_cuda:
-        _fail("topk_ids must be on the GPU")
-    if topk_ids.ndim != 2:
-        _fail("topk_ids must be [M, topk]")
+def _align(topk_ids: torch.Tensor, block_size: int, num_experts: int, with_offsets: bool):
+    """(sorted_ids, expert_ids, num_post, offsets or None, dropped or None)."""
     M, topk = topk_ids.shape
     em, nb = _lib.align_sizes(M, topk, num_experts, block_size)
     dev = topk_ids.device
@@ -187,34 +177,43 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     sorted_ids = torch.empty(em, dtype=torch.int32, device=dev)
     expert_ids = torch.empty(nb, dtype=torch.int32, device=dev)
     num_post = torch.empty(1, dtype=torch.int32, device=dev)
+    offsets = dropped = None
+    if with_offsets:
+        offsets = torch.empty(num_experts + 1, dtype=torch.int32, device=dev)
+        dropped = torch.empty(1, dtype=torch.int32, device=dev)
+    # Scratch of the many-workgroup sort of large batches (M=4096, top-10:
+    # 49.6 us on one workgroup with the router step, 29.1 with it); freed in stream order.
+    nbytes = _lib.align_scratch_size(M, topk, num_experts)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
     with torch.cuda.device(dev):
-        st = _lib.lib().w4a16_moe_align_block_size(
+        st = _lib.lib().w4a16_moe_align_block_size_ws(
             ids.data_ptr(), M, topk, num_experts, block_size, sorted_ids.data_ptr(),
-            expert_ids.data_ptr(), num_post.data_ptr(), None, None, _stream_ptr(dev))
+            expert_ids.data_ptr(), num_post.data_ptr(), _ptr(offsets), _ptr(dropped),
+            _ptr(scratch), nbytes, _stream_ptr(dev))
     _lib.check(st)
-    return sorted_ids, expert_ids, num_post
+    return sorted_ids, expert_ids, num_post, offsets, dropped
+
+
+def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: int):
+    """Sort token-slots by expert and pad each expert to a multiple of block_size.
+
+    Returns (sorted_token_ids int32[EM], expert_ids int32[EM/B],
+    num_tokens_post_padded int32[1]) with EM = round_up(M*topk + E*(B-1), B),
+    bit-identical to kernels/w4a16_moe.py:187-290.  One HIP launch (two from
+    8,192 pairs) on the current stream, no host synchronisation.
+    """
+    if not topk_ids.is_cuda:
+        _fail("topk_ids must be on the GPU")
+    if topk_ids.ndim != 2:
+        _fail("topk_ids must be [M, topk]")
+    return _align(topk_ids, block_size, num_experts, False)[:3]
 
 
 def moe_align_block_size_full(topk_ids: torch.Tensor, block_size: int, num_experts: int):
     """moe_align_block_size plus expert_offsets int32[E+1] and the dropped count."""
     if not topk_ids.is_cuda or topk_ids.ndim != 2:
         _fail("topk_ids must be a [M, topk] GPU tensor")
-    M, topk = topk_ids.shape
-    em, nb = _lib.align_sizes(M, topk, num_experts, block_size)
-    dev = topk_ids.device
-    ids = _ids_i32(topk_ids)
-    sorted_ids = torch.empty(em, dtype=torch.int32, device=dev)
-    expert_ids = torch.empty(nb, dtype=torch.int32, device=dev)
-    num_post = torch.empty(1, dtype=torch.int32, device=dev)
-    offsets = torch.empty(num_experts + 1, dtype=torch.int32, device=dev)
-    dropped = torch.empty(1, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
-        st = _lib.lib().w4a16_moe_align_block_size(
-            ids.data_ptr(), M, topk, num_experts, block_size, sorted_ids.data_ptr(),
-            expert_ids.data_ptr(), num_post.data_ptr(), offsets.data_ptr(),
-            dropped.data_ptr(), _stream_ptr(dev))
-    _lib.check(st)
-    return sorted_ids, expert_ids, num_post, offsets, dropped
+    return _align(topk_ids, block_size, num_experts, True)
 
 
 # ---------------------------------------------------------------------------

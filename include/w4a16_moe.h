@@ -112,7 +112,8 @@ int w4a16_moe_align_sizes(int64_t M, int64_t topk, int64_t num_experts,
  *   num_tokens_post_padded[1].
  * Optional outputs (may be NULL): expert_offsets[E+1] (exclusive prefix of
  * padded counts) and dropped[1] (pairs whose id is outside [0, E)).
- * One kernel launch on `stream`.
+ * One kernel launch on `stream`, by one workgroup;
+ * w4a16_moe_align_block_size_ws sorts large batches on many.
  */
 int w4a16_moe_align_block_size(const int32_t* topk_ids, int64_t M,
                                int64_t topk, int64_t num_experts,
@@ -121,6 +122,23 @@ int w4a16_moe_align_block_size(const int32_t* topk_ids, int64_t M,
                                int32_t* num_tokens_post_padded,
                                int32_t* expert_offsets, int32_t* dropped,
                                void* stream);
+
+/*
+ * The same with device scratch of w4a16_moe_align_scratch_size bytes (4-byte
+ * aligned; 0 bytes: none is used and `scratch` may be NULL): batches of 8,192
+ * pairs or more (E <= 512) then sort on one workgroup per 1,024 pairs, in two
+ * launches.  Same outputs, bit for bit.  The scratch need not be cleared and
+ * is free for other work after the call in stream order.
+ */
+int w4a16_moe_align_scratch_size(int64_t M, int64_t topk, int64_t num_experts,
+                                 size_t* bytes);
+int w4a16_moe_align_block_size_ws(const int32_t* topk_ids, int64_t M,
+                                  int64_t topk, int64_t num_experts,
+                                  int64_t block_size, int32_t* sorted_token_ids,
+                                  int32_t* expert_ids,
+                                  int32_t* num_tokens_post_padded,
+                                  int32_t* expert_offsets, int32_t* dropped,
+                                  void* scratch, size_t scratch_bytes, void* stream);
 
 /*
  * Device scratch needed by w4a16_moe_fused_experts (bytes, 256-aligned).

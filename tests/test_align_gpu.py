@@ -97,3 +97,32 @@ def test_align_int64_ids_and_plain_api(pkg, orc, dev):
     assert np.array_equal(s.cpu().numpy(), want[0])
     assert np.array_equal(e.cpu().numpy(), want[1])
     assert np.array_equal(n.cpu().numpy(), want[2])
+
+
+@pytest.mark.parametrize("M,topk,E", [(8191, 1, 64), (8192, 1, 64), (1025, 8, 512),
+                                      (4500, 2, 513), (5000, 10, 7)])
+@pytest.mark.parametrize("block", [1, 16, 48])
+def test_scratch_sort_equals_one_workgroup(pkg, orc, dev, M, topk, E, block):
+    """Around the many-workgroup sort's limits (8,192 pairs, 512 experts), with
+    ids outside [0, E): the call with scratch, the call without and the
+    oracle agree over the whole buffers."""
+    rng = np.random.default_rng(M + E)
+    ids = rng.integers(-1, E + 1, size=(M, topk)).astype(np.int32)
+    print(f"align scratch M={M} topk={topk} E={E} block={block}", flush=True)
+    got = _run(pkg, ids, block, E, dev)
+    _assert_exact(got, orc.moe_align_block_size(ids, block, E), f"M{M} E{E} B{block}")
+    L = pkg._lib
+    em, nb = L.align_sizes(M, topk, E, block)
+    t = torch.from_numpy(ids).to(dev)
+    s = torch.empty(em, dtype=torch.int32, device=dev)
+    e = torch.empty(nb, dtype=torch.int32, device=dev)
+    n = torch.empty(1, dtype=torch.int32, device=dev)
+    L.check(L.lib().w4a16_moe_align_block_size(
+        t.data_ptr(), M, topk, E, block, s.data_ptr(), e.data_ptr(), n.data_ptr(), None, None,
+        torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert np.array_equal(s.cpu().numpy(), got[0])
+    assert np.array_equal(e.cpu().numpy(), got[1])
+    assert np.array_equal(n.cpu().numpy(), got[2])
+    chunked = M * topk >= 8192 and E <= 512
+    assert (L.align_scratch_size(M, topk, E) > 0) == chunked
