@@ -152,15 +152,16 @@ int small_row_tiles(int64_t n_blocks, int64_t rows) {
 // fragments of a whole group do not fit the registers of taller tiles.
 constexpr int64_t kXTile32MaxPairs = 24;
 constexpr int kXTile128 = 48;
+constexpr int64_t kXTileMinPairs = 2;  // average pairs per expert they start at
 // Row tiles (`rows` outputs each) one workgroup of the exact-weight tiles runs
-// in turn: about 16 steps of 128 elements, so that short reductions do not
-// pay a workgroup's first loads for each row tile, with six workgroups per CU
+// in turn: about 32 steps of 128 elements, so that short reductions do not
+// pay a workgroup's first loads for each row tile, with seven workgroups per CU
 // left for balance.
 int xtile_row_tiles(int64_t n_out, int64_t kdim, int64_t rows, int64_t max_tiles) {
   const int64_t n_rt = (n_out + rows - 1) / rows;
   const int64_t steps = (kdim + 127) / 128;
-  const int64_t want = std::max<int64_t>(1, 16 / steps);
-  const int64_t fill = std::max<int64_t>(1, max_tiles * n_rt / (6 * kCUs));
+  const int64_t want = std::max<int64_t>(1, 32 / steps);
+  const int64_t fill = std::max<int64_t>(1, max_tiles * n_rt / (7 * kCUs));
   return (int)std::min<int64_t>(n_rt, std::min(want, fill));
 }
 // Average (token, slot) pairs per expert from which the built-in split sends
@@ -248,10 +249,16 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
   // multiple of 256, scales that are not 16-byte aligned, or by the tuning):
   // MFMA tiles of exact weights, any K and N the library takes.  The GEMV's
   // passes of four rows, which ran them before, cost a pass over the weights
-  // per four pairs: E=256, K=3072, N=128, 80 pairs per expert 1,272 -> 207 us
-  // per call; E=64, K=2048, N=1408, group 128, 73 pairs 1,351 -> 203 us.
-  L->xtile = !L->mfma && !L->route;
-  L->gemv = L->mfma ? L->gemv_max_tokens > 0 : L->route;
+  // per four pairs: E=256, K=3072, N=128, 80 pairs per expert 1,275 -> 175 us
+  // per call; E=64, K=2048, N=1408, group 128, 73 pairs 1,345 -> 191 us.
+  // Below two pairs per expert on average the GEMV over the sorted 16-slot
+  // blocks stays: its short work items fill the chip (E=128, top-4, K=1536,
+  // N=320: M=25 38.9 against 43.3 us, M=48 50.5 against 57.6, M=64 60.8
+  // against 57.6; E=256, top-10, K=3072, N=128: M=25 60.5 against 64.6, M=39
+  // 80.5 against 70.3).  Under skewed routing the tiles win everywhere (M=25
+  // 57 against 39 us), but the host does not see the routing.
+  L->xtile = !L->mfma && !L->route && (int64_t)n_tok >= kXTileMinPairs * E;
+  L->gemv = L->mfma ? L->gemv_max_tokens > 0 : !L->xtile;
   L->tc = T.tc;
   L->upw = T.upw;
   L->lpr = T.lpr;
@@ -281,7 +288,9 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
     L->row_tiles_w13 = xtile_row_tiles(N, K, 128, L->max_tiles);
     L->row_tiles_w2 = xtile_row_tiles(K, N, 256, L->max_tiles);
   }
-  L->max_gemv = L->mfma ? std::min<int64_t>(std::min<int64_t>(E, (int64_t)n_tok), L->nb) : 0;
+  L->max_gemv = L->mfma    ? std::min<int64_t>(std::min<int64_t>(E, (int64_t)n_tok), L->nb)
+                : L->xtile ? 0
+                           : std::min<int64_t>((int64_t)n_tok, L->nb);
   L->max_items = L->route ? (int64_t)n_tok : 0;
   L->token = L->route && M <= T.w2_fused_max_m && w2_token_fits((int)topk, (int)K, (int)N);
   L->partial_bf16 = M > kFp32PartialMaxM;
@@ -394,7 +403,7 @@ Work work_of(const Layout& L, void* ws_base) {
 // The GEMV launch of GEMM `mode` (0: w13, 1: w2).
 GemvLaunch gemv_args(const FusedArgs& a, const Layout& L, const Work& w, int mode) {
   GemvLaunch g{};
-  g.block_list = L.route ? nullptr : w.gemv_blocks;
+  g.block_list = L.mfma ? w.gemv_blocks : nullptr;
   g.sorted = w.sorted;
   g.expert_ids = w.eids;
   g.header = w.header;

@@ -165,8 +165,8 @@ struct GemvLaunch {
   int32_t group;
   int32_t max_blocks;      // upper bound of active blocks
   int32_t num_experts;
-  const int32_t* block_list;  // work item b is block block_list[b], b < header[3]
-                              // (not read by self-routing calls)
+  const int32_t* block_list;  // null: work item b is block b; else blocks
+                              // block_list[0 .. header[3])
   uint32_t nib_mask;          // set by the launcher (see gemv.hip)
   uint32_t nib_magic;
   // Self-routing (small batches, the align kernel is not run): when `ids`

@@ -336,8 +336,11 @@ __device__ __forceinline__ void gemv_item(const GemvLaunch a, int bid, u32x4_t* 
     if (MODE == 0 && a.route_items && slab0 == 0 && tid == 0) a.route_items[item] = e;
     if (e < 0) return;  // workgroup-uniform: every wave routes the same item
   } else {
-    if (item >= a.header[3]) return;
-    const int blk = a.block_list[item];
+    int blk = item;
+    if (a.block_list) {
+      if (item >= a.header[3]) return;
+      blk = a.block_list[item];
+    }
     if (blk * a.block >= a.header[0]) return;
     e = a.expert_ids[blk];
     if (e < 0) return;

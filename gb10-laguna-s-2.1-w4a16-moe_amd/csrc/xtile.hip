@@ -41,7 +41,6 @@
 
 namespace w4a16 {
 namespace {
-
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -97,10 +96,12 @@ __device__ __forceinline__ int frag_octet(int j, int q) {
   else return 4 * q + j;
 }
 
-// One tile of TB token blocks (16 slots each).  GS = log2(group / 32).  SV:
-// a row's scales are whole, aligned 16-byte pieces; else they are loaded one
-// by one, with indexes clamped to the row.
-template <int MODE, int GS, bool SV, int TB, class X>
+// One tile of TB token blocks (16 slots each).  GS = log2(group / 32).  SP:
+// scales per load: a row's scales are whole, aligned pieces of 8 (16 bytes) or
+// 4 (8 bytes), else they are loaded one by one.
+// kStaged = false: the reduction has at most two steps, which stay in the two
+// buffers: the loop loads no activations and needs no barrier.
+template <int MODE, int GS, int SP, int TB, class X, bool kStaged>
 __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, int nrt,
                                           const int* s_f, const float* s_wt, int count,
                                           unsigned char* lds) {
@@ -123,17 +124,19 @@ __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, 
 #pragma unroll
   for (int b = 0; b < TB; ++b) {
     int f = s_f[16 * b + at];
-    if (16 * b + at >= count) f = s_f[0];  // padding slots: any row, never stored
+    if (16 * b + at >= count) f = s_f[0];  // padding slots: a row to load, not used
     const int64_t row = MODE == 0 ? f / a.topk : f;
     arow[b] = reinterpret_cast<const char*>(a.act + row * a.ld_act);
   }
+  // Padding slots (of the last block) are zeros: their MFMAs draw less power.
+  const bool pad = 16 * (TB - 1) + at >= count;
   const int n_oct = a.kdim >> 3;
   // With two register sets in turn, a step's rows are written to LDS two
   // steps after their loads were issued: loads return in order, so the wait
   // for them leaves the weight loads of two steps in flight.  (Tall tiles of
   // the larger groups have registers for one set: one step.)
   constexpr int kSets = TB <= 2 ? 2 : 1;
-  constexpr bool kWhole = SV || GS == 2;  // K is a multiple of 128: no partial steps
+  constexpr bool kWhole = SP > 1 || GS == 2;  // K is a multiple of 128: no partial steps
   u32x4_t ars[kSets][TB];
   int ka = 0;  // local step of the next activation load
   bool ar_oks[kSets];
@@ -160,7 +163,8 @@ __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, 
   auto write_act = [&](const u32x4_t (&ar)[TB], bool ar_ok, int buf) {
 #pragma unroll
     for (int b = 0; b < TB; ++b) {
-      const u32x4_t d = kWhole || ar_ok ? ar[b] : u32x4_t{0u, 0u, 0u, 0u};
+      const bool ok = (kWhole || ar_ok) && (b < TB - 1 || !pad);
+      const u32x4_t d = ok ? ar[b] : u32x4_t{0u, 0u, 0u, 0u};
       u32x4_t p;
       p[0] = __builtin_amdgcn_perm(d[2], d[0], 0x05040100u);  // (x0, x4)
       p[1] = __builtin_amdgcn_perm(d[2], d[0], 0x07060302u);  // (x1, x5)
@@ -192,7 +196,7 @@ __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, 
   // 8 + l / 8), so that one instruction reads whole 128-byte lines, which the
   // launch never reads again: non-temporal, as the GEMV's.  (Lane l on row
   // l % 16, as the MFMA wants them, makes every lane a line of its own, and
-  // lines read in halves lose with the hint: see the launcher's figures.)
+  // lines read in halves lose with the hint: 210 against 286 us.)
   // The words go through this wave's own LDS to lane (n, q): 16-byte position
   // c of row m holds chunk c ^ ((m / 4) % 4) of its step, which spreads a
   // read of 16 rows over all banks; the 128 bytes between the steps' halves
@@ -256,7 +260,7 @@ __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, 
   // wave's own LDS, loaded a window ahead.  Loading each step's few scales on
   // their own cost a cache line per row and step (w13 of 256 experts with 10
   // pairs each, K=3072, N=1024: 302 us, 196 without the scale loads).
-  constexpr int kWin = SV ? X::kWin : 8;  // scales of a row per window
+  constexpr int kWin = SP == 8 ? X::kWin : 8;  // scales of a row per window
   constexpr int kWinSteps = kWin / kSc;   // steps per window
   constexpr int kPc = kWin / 8;           // 16-byte pieces of a row's window
   const int n_win = (T + kWinSteps - 1) / kWinSteps;
@@ -264,13 +268,22 @@ __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, 
   u32x4_t sreg[kPc];
   int rt_s = rt0, w_s = 0;  // row tile and window of the next scale load
   auto load_scales = [&]() {
-    if constexpr (SV) {  // rows of whole 16-byte pieces: piece lane % kPc
+    if constexpr (SP == 8) {  // piece lane % kPc of rows lane / kPc, ...
 #pragma unroll
       for (int i = 0; i < kPc; ++i) {
         const int m = (64 / kPc) * i + lane / kPc;  // row of the wave: block m / 16
         const uint32_t r = (uint32_t)wrow(rt_s, m >> 4, m & 15);
         const uint32_t c = (uint32_t)min(kPc * w_s + lane % kPc, (gpr >> 3) - 1);
         sreg[i] = *reinterpret_cast<const u32x4_t*>(sexp + (r * (uint32_t)gpr * 2u + c * 16u));
+      }
+    } else if constexpr (SP == 4) {  // one row per lane
+      const uint32_t r = (uint32_t)wrow(rt_s, q, n);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t c = (uint32_t)min(2 * w_s + i, (gpr >> 2) - 1);
+        const u32x2_t v =
+            *reinterpret_cast<const u32x2_t*>(sexp + (r * (uint32_t)gpr * 2u + c * 8u));
+        sreg[0][2 * i] = v[0], sreg[0][2 * i + 1] = v[1];
       }
     } else {  // any alignment: one row per lane
       const uint32_t r = (uint32_t)wrow(rt_s, q, n);
@@ -419,32 +432,30 @@ __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, 
   // Outputs of row tile rt: lane (q, n) holds tokens 16 b + 4 q + r of its
   // rows; its neighbouring rows make one store per token.
   auto write_out = [&](int rt) {
+    const int first = (rt * kWaves + wid) * (MODE == 0 ? 32 : 64) + (MODE == 0 ? 2 : 4) * n;
+    const bool rows_ok = first < a.n_out;
+    const int elt = MODE == 1 && !a.partial_bf16 ? 4 : 2;
+    char* const base = static_cast<char*>(a.out) + (int64_t)first * elt;
+    const int pitch = a.n_out * elt;
 #pragma unroll
     for (int b = 0; b < TB; ++b) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int t = 16 * b + 4 * q + r;
-        const int f = s_f[t];
+        char* const o = base + (int64_t)s_f[t] * pitch;
         if (MODE == 0) {
-          const int col = (rt * kWaves + wid) * 32 + 2 * n;
           const float h0 = silu(acc[0][b][r]) * acc[2][b][r];
           const float h1 = silu(acc[1][b][r]) * acc[3][b][r];
-          if (t < count && col < a.n_out)
-            *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(a.out) +
-                                         (int64_t)f * a.n_out + col) = pack2(h0, h1);
+          if (t < count && rows_ok) *reinterpret_cast<uint32_t*>(o) = pack2(h0, h1);
         } else {
-          const int row = (rt * kWaves + wid) * 64 + 4 * n;
           const float wt = s_wt[t];
           const float v0 = acc[0][b][r] * wt, v1 = acc[1][b][r] * wt;
           const float v2 = acc[2][b][r] * wt, v3 = acc[3][b][r] * wt;
-          if (t < count && row < a.n_out) {
-            const int64_t o = (int64_t)f * a.n_out + row;
+          if (t < count && rows_ok) {
             if (a.partial_bf16)
-              *reinterpret_cast<u32x2_t*>(static_cast<uint16_t*>(a.out) + o) =
-                  u32x2_t{pack2(v0, v1), pack2(v2, v3)};
+              *reinterpret_cast<u32x2_t*>(o) = u32x2_t{pack2(v0, v1), pack2(v2, v3)};
             else
-              *reinterpret_cast<f32x4_t*>(static_cast<float*>(a.out) + o) =
-                  f32x4_t{v0, v1, v2, v3};
+              *reinterpret_cast<f32x4_t*>(o) = f32x4_t{v0, v1, v2, v3};
           }
         }
       }
@@ -457,63 +468,74 @@ __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, 
   // has read its weights, stores the next pair's and loads those of the pair
   // after.  The loads are unconditional, so that the compiler's waits leave
   // the newer ones in flight on every path.
+  static_assert(kWinSteps % 2 == 0, "scale windows end with a pair of steps");
   load_scales();
   load_w();
   load_act(ars[0], ar_oks[0]);
   if (kSets == 2) load_act(ars[kSets - 1], ar_oks[kSets - 1]);
-  store_w();
-  load_w();
+  // (in the order of the loop's second step: the compiler's waits are the
+  // strictest over the ways into the loop, and with the weights issued before
+  // the activations here each step waited for the weights just issued)
   write_act(ars[0], ar_oks[0], 0);
   load_act(ars[0], ar_oks[0]);
+  store_scales();
+  store_w();
+  load_w();
+  load_scales();
   read_w(0);
+  if (!kStaged && T == 2) write_act(ars[kSets - 1], ar_oks[kSets - 1], kBuf);
   lds_barrier();
   int k = 0, ks = 0, rt = rt0;
   for (int gp = nrt * TP; gp > 0; --gp) {
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      constexpr int kS1 = kSets - 1;
-      write_act(ars[(p + 1) & kS1], ar_oks[(p + 1) & kS1], p ? 0 : kBuf);
-      load_act(ars[(p + 1) & kS1], ar_oks[(p + 1) & kS1]);
+      if constexpr (kStaged) {
+        constexpr int kS1 = kSets - 1;
+        write_act(ars[(p + 1) & kS1], ar_oks[(p + 1) & kS1], p ? 0 : kBuf);
+        load_act(ars[(p + 1) & kS1], ar_oks[(p + 1) & kS1]);
+      }
       if (p == 1) {
         store_w();
         load_w();
       }
       if (p == 0 || k < T) {
-        if (ks == 0) {
-          store_scales();
-          load_scales();
-        }
         read_scales(ks);
         compute(p ? kBuf : 0);
-        ks = ks + 1 == kWinSteps ? 0 : ks + 1;
       }
-      ++k;
+      ++k, ++ks;
       if (p == 1 && k >= T) {
         write_out(rt);
         clear();
-        k = ks = 0;
+        k = 0, ks = kWinSteps;
         ++rt;
       }
+      // the next scale window, behind the newest weight loads (windows are an
+      // even number of steps)
+      if (p == 1 && ks == kWinSteps) {
+        store_scales();
+        load_scales();
+        ks = 0;
+      }
       read_w(p ? 0 : 1);
-      lds_barrier();
+      if constexpr (kStaged) lds_barrier();
     }
   }
 }
 
-template <int MODE, int GS, bool SV, class X>
+template <int MODE, int GS, int SP, class X>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void xtile_kernel(const XtileLaunch a) {
   __shared__ __align__(16) unsigned char lds[X::kLds];
   __shared__ int s_f[X::kTileM];
   __shared__ float s_wt[X::kTileM];
   __shared__ int s_count;
-  static_assert(X::kTileM <= 64, "one wave lists the tile's pairs");
+  const int bid = (int)blockIdx.x;
   const int rows_per_tile = MODE == 0 ? kWaves * 32 : kWaves * 64;
   const int n_rt = (a.n_out + rows_per_tile - 1) / rows_per_tile;
   const int items = (n_rt + a.row_tiles - 1) / a.row_tiles;
   // Tiles are dealt over the 8 XCDs in rounds that alternate direction, and
   // the items of one tile run back to back on its XCD (as in mfma_item).
-  const int xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
+  const int xcd = bid % kXcds, slot = bid / kXcds;
   const int round = slot / items;
   const int tile = kXcds * round + ((round & 1) ? kXcds - 1 - xcd : xcd);
   if (tile >= a.header[2]) return;
@@ -523,6 +545,7 @@ void xtile_kernel(const XtileLaunch a) {
   const int start = (info & 0x0FFFFFFF) << 4;
   const int blocks = min(info >> 28, X::kTBMax);
   const int e = __builtin_amdgcn_readfirstlane(a.expert_ids[start >> 4]);
+  static_assert(X::kTileM <= 64, "one wave lists the tile's pairs");
   if (threadIdx.x < 64) {  // the tile's pairs are a prefix of its slots
     const int i = threadIdx.x;
     const int f = i < 16 * blocks ? a.sorted[start + i] : a.n_tok;
@@ -536,10 +559,16 @@ void xtile_kernel(const XtileLaunch a) {
   }
   __syncthreads();
   const int count = __builtin_amdgcn_readfirstlane(s_count);
+  // (w2 of a layer sliced to N <= 256; a hidden size is not that short)
+  const bool short_k = a.kdim <= 256;
 #define W4A16_XTILE(TB_)                                                                   \
   case TB_:                                                                                \
-    if constexpr (TB_ <= X::kTBMax)                                                        \
-      run_xtile<MODE, GS, SV, TB_, X>(a, e, rt0, nrt, s_f, s_wt, count, lds);              \
+    if constexpr (TB_ <= X::kTBMax) {                                                      \
+      if (MODE == 1 && short_k)                                                            \
+        run_xtile<MODE, GS, SP, TB_, X, MODE == 0>(a, e, rt0, nrt, s_f, s_wt, count, lds); \
+      else                                                                                 \
+        run_xtile<MODE, GS, SP, TB_, X, true>(a, e, rt0, nrt, s_f, s_wt, count, lds);      \
+    }                                                                                      \
     break;
   switch ((count + 15) >> 4) {
     W4A16_XTILE(1)
@@ -551,22 +580,30 @@ void xtile_kernel(const XtileLaunch a) {
 #undef W4A16_XTILE
 }
 
-template <int MODE, class X>
-void launch_geo(const XtileLaunch& a, dim3 g, bool sv, hipStream_t stream) {
+template <int MODE, int GS, class X>
+void launch_sp(const XtileLaunch& a, dim3 g, hipStream_t stream) {
   const dim3 b(kWaves * 64);
-#define W4A16_XTILE(GS_)                                                                   \
-  if (sv)                                                                                  \
-    hipLaunchKernelGGL((xtile_kernel<MODE, GS_, true, X>), g, b, 0, stream, a);            \
-  else                                                                                     \
-    hipLaunchKernelGGL((xtile_kernel<MODE, GS_, false, X>), g, b, 0, stream, a);
-  if (a.group == 32) {
-    W4A16_XTILE(0)
-  } else if (a.group == 64) {
-    W4A16_XTILE(1)
-  } else {
-    W4A16_XTILE(2)
-  }
-#undef W4A16_XTILE
+  const int gpr = a.kdim / a.group;
+  const uintptr_t s = reinterpret_cast<uintptr_t>(a.s);
+  if (gpr % 8 == 0 && s % 16 == 0)
+    hipLaunchKernelGGL((xtile_kernel<MODE, GS, 8, X>), g, b, 0, stream, a);
+  else if (gpr % 4 == 0 && s % 8 == 0)
+    hipLaunchKernelGGL((xtile_kernel<MODE, GS, 4, X>), g, b, 0, stream, a);
+  else
+    hipLaunchKernelGGL((xtile_kernel<MODE, GS, 1, X>), g, b, 0, stream, a);
+}
+
+// Tiles of at most 32 slots, else of 64 (48 for groups of 128).
+template <int MODE, int GS>
+hipError_t launch_geo(const XtileLaunch& a, dim3 g, hipStream_t stream) {
+  using Tall = XGeo<GS == 2 ? 3 : 4>;
+  if (a.tile_m <= XGeo<2>::kTileM)
+    launch_sp<MODE, GS, XGeo<2>>(a, g, stream);
+  else if (a.tile_m <= Tall::kTileM)
+    launch_sp<MODE, GS, Tall>(a, g, stream);
+  else
+    return hipErrorInvalidValue;
+  return hipGetLastError();
 }
 
 template <int MODE>
@@ -575,8 +612,7 @@ hipError_t launch_xtile(const XtileLaunch& a_in, hipStream_t stream) {
   a.nib_mask = 0x000F000Fu;
   a.nib_magic = 0x43004300u;  // bf16 (128, 128)
   if (a.kdim < 32 || a.kdim % 32 != 0 || a.n_out < 32 || a.n_out % 32 != 0 || a.row_tiles < 1 ||
-      a.max_tiles < 0 ||
-      a.tile_m < 16 || a.tile_m > kXTileM || (a.group != 32 && a.group != 64 && a.group != 128))
+      a.max_tiles < 0 || a.tile_m < 16)
     return hipErrorInvalidValue;
   const int rows_per_tile = MODE == 0 ? kWaves * 32 : kWaves * 64;
   const int n_rt = (a.n_out + rows_per_tile - 1) / rows_per_tile;
@@ -585,15 +621,12 @@ hipError_t launch_xtile(const XtileLaunch& a_in, hipStream_t stream) {
   if (grid <= 0) return hipSuccess;
   if (grid > INT32_MAX) return hipErrorInvalidValue;
   const dim3 g((unsigned)grid);
-  // scale rows of whole, aligned 16-byte pieces
-  const bool sv = a.kdim / a.group % 8 == 0 && reinterpret_cast<uintptr_t>(a.s) % 16 == 0;
-  if (a.tile_m <= XGeo<2>::kTileM)
-    launch_geo<MODE, XGeo<2>>(a, g, sv, stream);
-  else if (a.tile_m <= XGeo<3>::kTileM)
-    launch_geo<MODE, XGeo<3>>(a, g, sv, stream);
-  else
-    launch_geo<MODE, XGeo<4>>(a, g, sv, stream);
-  return hipGetLastError();
+  switch (a.group) {
+    case 32: return launch_geo<MODE, 0>(a, g, stream);
+    case 64: return launch_geo<MODE, 1>(a, g, stream);
+    case 128: return launch_geo<MODE, 2>(a, g, stream);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 }  // namespace

@@ -247,9 +247,9 @@ int w4a16_moe_dropped_pairs(const void* workspace, int32_t* count,
  *   gemv_only_max_m       calls with M <= this run every expert on exact
  *                         weights: the GEMV kernels routing themselves (up to
  *                         256 pairs, when it fits in LDS), else the sort and
- *                         MFMA tiles of exact weights (so do calls whose N or
- *                         K is no multiple of 256 or whose scales are not
- *                         16-byte aligned);
+ *                         MFMA tiles of exact weights (so do larger calls
+ *                         whose N or K is no multiple of 256 or whose scales
+ *                         are not 16-byte aligned);
  *   gemv_max_tokens       larger calls (N, K multiples of 256) send experts
  *                         with more (token, slot) pairs than this (0..15) to
  *                         the MFMA kernels, the others to the GEMV kernels;

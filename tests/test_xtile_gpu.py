@@ -3,7 +3,7 @@ edges of their tiles, row tiles, steps and scale windows.
 
 The calls are the ones that reach them: N or K no multiple of 256, scales that
 are not 16-byte aligned, or a tuning that keeps every expert on exact weights,
-with more than 256 pairs (or more than 24 tokens).  No weight is rounded, so
+with too many pairs to route themselves and at least two per expert.  No weight is rounded, so
 the bars are the tight ones of test_fused_gpu.py for exact experts.
 """
 
@@ -92,7 +92,7 @@ def test_unaligned_scales_and_fp32_partials(pkg, orc, synth, dev, K, N, group):
 def test_workspace_no_larger_than_the_sorted_blocks(pkg):
     """The tile list holds at most one entry per sorted 16-slot block."""
     L = pkg._lib
-    for M, topk, E in ((30, 10, 256), (777, 6, 64), (2048, 10, 256), (100, 4, 1024)):
+    for M, topk, E in ((30, 10, 256), (50, 10, 256), (777, 6, 64), (2048, 10, 256), (400, 4, 1024)):
         off = L.workspace_layout(M, topk, E, 128, 1056, 32)
         _, nb = L.align_sizes(M, topk, E, 16)
         span = off[L.WS_GEMV_BLOCKS] - off[L.WS_TILES]
