@@ -9,12 +9,15 @@ are valid here.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 from pathlib import Path
 
 import torch  # noqa: F401  (loads torch's HIP runtime first, see above)
 
 LIB_PATH = Path(__file__).resolve().parent / "libw4a16moe.so"
+FAST_PATH = LIB_PATH.parent / "w4a16_fastcall.so"
 
 W4A16_OK = 0
 W4A16_ERR_NULL_POINTER = 1
@@ -76,6 +79,7 @@ _i64 = ctypes.c_int64
 _vp = ctypes.c_void_p
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
+_fast = None
 
 
 class LibraryNotBuilt(RuntimeError):
@@ -163,6 +167,27 @@ def lib() -> ctypes.CDLL:
                 raise RuntimeError("libw4a16moe.so ABI version mismatch")
             _lib = handle
     return _lib
+
+
+def fast():
+    """The native call path (csrc/fastcall.cpp); raises LibraryNotBuilt if it
+    is missing."""
+    global _fast
+    if _fast is not None:
+        return _fast
+    lib()
+    with _lock:
+        if _fast is None:
+            if not FAST_PATH.exists():
+                raise LibraryNotBuilt(
+                    f"{FAST_PATH} is missing: build it with __graft_entry__.build()")
+            loader = importlib.machinery.ExtensionFileLoader("w4a16_fastcall", str(FAST_PATH))
+            spec = importlib.util.spec_from_file_location("w4a16_fastcall", FAST_PATH,
+                                                          loader=loader)
+            mod = importlib.util.module_from_spec(spec)
+            loader.exec_module(mod)
+            _fast = mod
+    return _fast
 
 
 def strerror(status: int) -> str:

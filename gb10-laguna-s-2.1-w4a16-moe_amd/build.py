@@ -19,6 +19,8 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_NAME = "libw4a16moe.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+FAST_SRC = CSRC / "fastcall.cpp"
+FAST_PATH = PKG_DIR / "w4a16_fastcall.so"
 OFFLOAD_ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -80,5 +82,29 @@ def build(verbose: bool = False) -> Path:
     return LIB_PATH
 
 
+def build_fastcall(verbose: bool = False) -> Path:
+    """Compile the host-side call path (a CPython module over torch's C++
+    headers, linked to LIB_PATH beside it) into FAST_PATH."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    inc = [*cpp_extension.include_paths(device_type="cuda"), sysconfig.get_paths()["include"]]
+    libs = cpp_extension.library_paths(device_type="cuda")
+    with tempfile.TemporaryDirectory(dir=PKG_DIR) as tmp:
+        so = Path(tmp) / FAST_PATH.name
+        _run([shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+              "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+              *(f"-isystem{d}" for d in inc), str(FAST_SRC), "-o", str(so),
+              f"-L{PKG_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN",
+              *(f"-L{d}" for d in libs), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+              "-lc10_hip"], verbose)
+        os.replace(so, FAST_PATH)
+    return FAST_PATH
+
+
 if __name__ == "__main__":
     print(build(verbose=True))
+    print(build_fastcall(verbose=True))

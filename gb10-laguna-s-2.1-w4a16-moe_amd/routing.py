@@ -31,6 +31,12 @@ def router_topk_softmax(router_logits: torch.Tensor, topk: int, renormalize: boo
     Returns ``(topk_weights fp32 [M, topk], topk_ids int32 [M, topk])``; ids
     are ordered by descending logit, equal logits by ascending expert index.
     """
+    if out is None:  # the native path takes the ordinary calls
+        got = _lib.fast().router(router_logits, topk, renormalize)
+        if got is not None:
+            if type(got) is int:
+                _lib.check(got)
+            return got
     if router_logits.dim() != 2:
         raise _lib.W4A16Error("router_logits must be [M, E]")
     if router_logits.dtype not in _DTYPES:

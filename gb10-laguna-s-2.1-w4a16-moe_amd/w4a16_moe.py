@@ -20,6 +20,7 @@ Differences from the reference, all deliberate:
 from __future__ import annotations
 
 import ctypes
+import os
 import threading
 
 import torch
@@ -34,6 +35,7 @@ BLOCK_M = 16
 BLOCK_N = 64
 BLOCK_K = 64
 
+_TUNING_ENV = ("W4A16_MOE_TUNING", "W4A16_MOE_CONFIG_DIR")
 
 
 class WorkspacePool:
@@ -59,12 +61,13 @@ class WorkspacePool:
     the life of the process.
     """
 
-    def __init__(self, alloc=None):
+    def __init__(self, alloc=None, on_clear=None):
         self._alloc = alloc or (lambda nbytes, device: torch.empty(
             nbytes, dtype=torch.uint8, device=device))
         self._bufs: dict[tuple, torch.Tensor] = {}
         self._retired: list[torch.Tensor] = []  # capture buffers outgrown in their capture
         self._lock = threading.Lock()
+        self._on_clear = on_clear  # called when every buffer is dropped
 
     def get(self, device, stream: int, nbytes: int, capture_id: int = 0) -> torch.Tensor:
         """A workspace of at least `nbytes` for a call on `stream`, under the
@@ -106,9 +109,11 @@ class WorkspacePool:
         with self._lock:
             self._bufs.clear()
             self._retired.clear()
+            if self._on_clear is not None:
+                self._on_clear()
 
 
-_WS_POOL = WorkspacePool()
+_WS_POOL = WorkspacePool(on_clear=lambda: _lib.fast().clear_workspaces())
 
 
 def release_graph_workspaces() -> None:
@@ -202,6 +207,11 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     bit-identical to kernels/w4a16_moe.py:187-290.  One HIP launch (two from
     8,192 pairs) on the current stream, no host synchronisation.
     """
+    got = _lib.fast().align(topk_ids, block_size, num_experts)
+    if got is not None:
+        if type(got) is int:
+            _lib.check(got)
+        return got
     if not topk_ids.is_cuda:
         _fail("topk_ids must be on the GPU")
     if topk_ids.ndim != 2:
@@ -238,7 +248,22 @@ def _workspace(device: torch.device, M: int, topk: int, E: int, N: int, K: int,
     nbytes = _lib.workspace_size_ex(M, topk, E, N, K, group, ts)
     stream = _stream_ptr(device)
     cap = _lib.capture_id(stream) if torch.cuda.is_current_stream_capturing() else 0
-    return _WS_POOL.get(device, stream, nbytes, capture_id=cap)
+    ws = _WS_POOL.get(device, stream, nbytes, capture_id=cap)
+    if not cap and device.index is not None:  # the native call path's view of the pool
+        _lib.fast().set_workspace(device.index, stream, ws)
+    return ws
+
+
+def _register_plan(p: "_Prepared") -> None:
+    """Tell the native call path (csrc/fastcall.cpp) how a call of this shape
+    runs when the caller passes no tuning.  It does not take calls while a
+    tuning environment variable is set, so none may enter here."""
+    if p.device.index is None or any(os.environ.get(v) for v in _TUNING_ENV):
+        return
+    ts = None if p.tuning is None else p.tuning.to_struct()
+    nbytes = _lib.workspace_size_ex(p.M, p.topk, p.E, p.N, p.K, p.group, ts)
+    fields = None if ts is None else tuple(int(getattr(ts, f)) for f, _ in ts._fields_)
+    _lib.fast().set_plan(p.device.index, p.M, p.topk, p.E, p.N, p.K, p.group, nbytes, fields)
 
 
 class _Prepared:
@@ -361,6 +386,13 @@ def fused_experts_w4a16(
     per-shape workspace exists).
     """
     del block_m, block_n, block_k
+    if tuning is None:  # the native path takes the calls it knows how to run
+        out = _lib.fast().fused(hidden, w1_q, w2_q, w1_scale, w2_scale, topk_weights, topk_ids,
+                                group_size)
+        if out is not None:
+            if type(out) is int:
+                _lib.check(out)
+            return out
     p = _prepare(hidden, w1_q, w2_q, w1_scale, w2_scale, topk_weights, topk_ids,
                  group_size)
     out = torch.empty((p.M, p.K), dtype=torch.bfloat16, device=p.device)
@@ -371,6 +403,8 @@ def fused_experts_w4a16(
     with torch.cuda.device(p.device):
         st = _lib.lib().w4a16_moe_fused_experts_ex(*_fused_args(p, out, ws), _tuning_ptr(p))
     _lib.check(st)
+    if tuning is None:
+        _register_plan(p)
     return out
 
 

@@ -1,0 +1,158 @@
+"""The native call path (csrc/fastcall.cpp): the calls it takes give the Python
+path's bits, and it leaves every other call to that path."""
+
+from __future__ import annotations
+
+import threading
+
+import pytest
+import torch
+
+from test_fused_gpu import _make
+
+
+@pytest.fixture(autouse=True)
+def no_tuning_variables(monkeypatch):
+    """The native path takes no calls while they are set (conftest.py does)."""
+    for var in ("W4A16_MOE_TUNING", "W4A16_MOE_CONFIG_DIR"):
+        monkeypatch.delenv(var, raising=False)
+
+
+def test_host_tensors_are_left_alone(pkg):
+    f = pkg._lib.fast()
+    t = torch.zeros(2, 2)
+    assert f.fused(t, t, t, t, t, t, t, 32) is None
+    assert f.router(t, 1, True) is None
+    assert f.align(t, 16, 4) is None
+    with pytest.raises(pkg._lib.W4A16Error):
+        pkg.fused_experts_w4a16(t, t, t, t, t, t, t)
+
+
+SHAPES = [(16, 4, 512, 256, 32, 6), (16, 4, 512, 256, 64, 40), (8, 2, 96, 160, 32, 90),
+          (256, 10, 3072, 1024, 32, 1)]
+
+
+def _bits(t):
+    return t.view(torch.int16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,topk,K,N,group,M", SHAPES)
+def test_same_bits_as_the_python_path(pkg, synth, dev, monkeypatch, E, topk, K, N, group, M):
+    shape = synth.LayerShape(E=E, topk=topk, K=K, N=N, group=group)
+    w13, w2, s13, s2, x, tw, ti = _make(synth, shape, M, dev, seed=M)
+    f = pkg._lib.fast()
+    f.clear_plans()
+    args = (x, w13, w2, s13, s2, tw, ti, group)
+    assert f.fused(*args) is None  # no plan yet
+    first = pkg.fused_experts_w4a16(*args)
+    fast = f.fused(*args)
+    assert isinstance(fast, torch.Tensor) and fast.shape == first.shape
+    assert torch.equal(_bits(fast), _bits(first))
+    wide = torch.zeros(M, K + 64, dtype=torch.bfloat16, device=dev)
+    wide[:, 32: 32 + K] = x
+    forms = [(wide[:, 32: 32 + K], w13.view(torch.uint8), w2.view(torch.uint8), s13, s2, tw,
+              ti.to(torch.int64), group),
+             (x, w13, w2, s13, s2, tw.t().contiguous().t(), ti.t().contiguous().t(), group)]
+    for a in forms:
+        assert torch.equal(_bits(f.fused(*a)), _bits(first))
+    # calls of a form or a moment it does not know
+    odd = torch.zeros(M, K + 4, dtype=torch.bfloat16, device=dev)[:, :K]  # row stride
+    assert f.fused(odd, *args[1:]) is None or odd.stride(0) % 8 == 0
+    assert f.fused(x.float(), *args[1:]) is None
+    assert f.fused(x, w13, w2, s13[:, ::2], s2, tw, ti, group) is None
+    assert f.fused(x, w13, w2, s13, s2, tw[:, :1], ti, group) is None
+    assert f.fused(x[:0], w13, w2, s13, s2, tw[:0], ti[:0], group) is None
+    assert f.fused(x.as_subclass(type("Sub", (torch.Tensor,), {})), *args[1:]) is None
+    for var in ("W4A16_MOE_TUNING", "W4A16_MOE_CONFIG_DIR"):
+        monkeypatch.setenv(var, "default")
+        assert f.fused(*args) is None
+        monkeypatch.delenv(var)
+    with pytest.raises(pkg._lib.W4A16Error):
+        pkg.fused_experts_w4a16(x, w13, w2, s13, s2, tw[:, :1], ti, group)
+    with torch.device("cuda:0"):  # a torch-function mode
+        assert f.fused(*args) is None
+
+
+@pytest.mark.gpu
+def test_streams_threads_and_growth(pkg, synth, dev):
+    """A stream seen for the first time goes through the Python path, which
+    gives it a workspace; threads on streams of their own then run at once;
+    a larger call grows the buffer both paths use."""
+    shape = synth.LayerShape(E=16, topk=4, K=512, N=256, group=32)
+    w = synth.make_weights(shape, dev, seed=1)
+    ins = []
+    for M in (8, 40, 300):
+        x = synth.make_hidden(M, shape.K, dev, seed=M)
+        tw, ti = synth.make_routing(M, shape.E, shape.topk, dev, seed=M)
+        ins.append((x, *w, tw, ti, 32))
+    want = [pkg.fused_experts_w4a16(*a) for a in ins]
+    torch.cuda.synchronize()
+    bad = []
+
+    def worker():
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            if pkg._lib.fast().fused(*ins[0]) is not None:
+                bad.append("a new stream has no workspace")
+            for _ in range(20):
+                for a, e in zip(ins, want):
+                    if not torch.equal(_bits(pkg.fused_experts_w4a16(*a)), _bits(e)):
+                        bad.append("bits")
+            ws, _ = pkg.workspace_tensor(ins[2][0], ins[2][6], w[0], w[1])
+            if pkg._lib.fast().fused(*ins[2]) is None:
+                bad.append("not taken")
+        s.synchronize()
+
+    threads = [threading.Thread(target=worker) for _ in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad
+
+
+@pytest.mark.gpu
+def test_capture_uses_the_captures_own_workspace(pkg, synth, dev):
+    shape = synth.LayerShape(E=16, topk=4, K=512, N=256, group=32)
+    w13, w2, s13, s2, x, tw, ti = _make(synth, shape, 40, dev, seed=3)
+    args = (x, w13, w2, s13, s2, tw, ti, 32)
+    want = pkg.fused_experts_w4a16(*args)
+    torch.cuda.synchronize()
+    taken = []
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        taken.append(pkg._lib.fast().fused(*args))
+        out = pkg.fused_experts_w4a16(*args)
+    assert taken == [None]
+    for _ in range(3):
+        out.zero_()
+        pkg.fused_experts_w4a16(*args)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(_bits(out), _bits(want))
+    del g
+    pkg.release_graph_workspaces()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 7, 900])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_router_and_align(pkg, dev, M, dtype):
+    g = torch.Generator(device=dev).manual_seed(M)
+    logits = torch.randn((M, 64), generator=g, device=dev).to(dtype)
+    f = pkg._lib.fast()
+    w, ids = f.router(logits, 10, True)
+    w2, ids2 = torch.empty_like(w), torch.empty_like(ids)
+    pkg.router_topk_softmax(logits, 10, out=(w2, ids2))  # the Python path
+    assert torch.equal(w, w2) and torch.equal(ids, ids2)
+    assert f.router(logits.t().contiguous().t(), 10, True) is None or M == 1
+    with pytest.raises(pkg._lib.W4A16Error):
+        pkg.router_topk_softmax(logits, 65)
+    got = f.align(ids, 16, 64)
+    want = pkg.moe_align_block_size_full(ids, 16, 64)[:3]
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert all(torch.equal(a, b) for a, b in zip(f.align(ids.to(torch.int64), 16, 64), want))
+    with pytest.raises(pkg._lib.W4A16Error):
+        pkg.moe_align_block_size(ids, 0, 64)
