@@ -152,6 +152,19 @@ int small_row_tiles(int64_t n_blocks, int64_t rows) {
 // fragments of a whole group do not fit the registers of taller tiles.
 constexpr int64_t kXTile32MaxPairs = 24;
 constexpr int kXTile128 = 48;
+// Pairs from which the sort and the exact-weight tiles beat the self-routed
+// GEMV: 2.5 per expert, and with few experts (whose tiles fill less of the
+// chip) 4.5 per expert or 72 in all.  Uniform routing, GEMV against tiles:
+// E=64, top-8, K=2048, N=768 M=16 51 / 54 us, M=20 55 / 55, M=24 65 / 56;
+// E=32, top-4 M=16 36 / 39, M=20 43 / 39; E=16, top-4, N=1024 M=16 40 / 43,
+// M=20 46 / 43; E=8, top-2, K=4096, N=1344 M=16 59 / 66, M=20 75 / 66.  Skewed
+// routing: the tiles from M=12 (E=64 M=24 84 / 43 us).  Layers of fewer than
+// 2^25 elements per projection are read in less time than the sort takes
+// (E=32, K=1024, N=512, M=24 26 / 31 us) and stay on the GEMV.
+bool many_pairs(int64_t n_tok, int64_t E, int64_t N, int64_t K) {
+  return 2 * n_tok >= 5 * E && n_tok >= std::min<int64_t>(9 * E / 2, 72) &&
+         E * N * K >= (int64_t)1 << 25;
+}
 constexpr int64_t kXTileMinPairs = 2;  // average pairs per expert they start at
 // Row tiles (`rows` outputs each) one workgroup of the exact-weight tiles runs
 // in turn: about 32 steps of 128 elements, so that short reductions do not
@@ -242,8 +255,10 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
   // every expert goes to the MFMA kernels and the GEMV launches are skipped.
   if (L->mfma && T.auto_split && (int64_t)n_tok >= kAllMfmaMinPairs * E) L->gemv_max_tokens = 0;
   // Small batches: the GEMV kernels route themselves from topk_ids (work
-  // item = one routed expert), so the align kernel is not run.
+  // item = one routed expert), so the align kernel is not run -- but not once
+  // their experts hold many pairs, whose passes of four add up.
   L->route = !L->mfma && M >= 1 && M <= T.gemv_only_max_m &&
+             !(M > T.w2_fused_max_m && many_pairs((int64_t)n_tok, E, N, K)) &&
              gemv_route_fits((int)n_tok, (int)E, (int)K, (int)N);
   // Every other call that keeps all experts on exact weights (K or N no
   // multiple of 256, scales that are not 16-byte aligned, or by the tuning):
