@@ -97,3 +97,25 @@ def test_workspace_no_larger_than_the_sorted_blocks(pkg):
         _, nb = L.align_sizes(M, topk, E, 16)
         span = off[L.WS_GEMV_BLOCKS] - off[L.WS_TILES]
         assert span <= (4 * min(nb, M * topk) + 255) // 256 * 256
+
+
+@pytest.mark.parametrize("K,N,group,M", [(1056, 704, 32, 120), (512, 128, 64, 300)])
+def test_graph_replay(pkg, synth, dev, K, N, group, M):
+    shape = synth.LayerShape(E=10, topk=3, K=K, N=N, group=group)
+    w13, w2, s13, s2, x, tw, ti = _make(synth, shape, M, dev, seed=M)
+    args = (w13, w2, s13, s2, tw, ti, group)
+    eager = pkg.fused_experts_w4a16(x, *args)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = pkg.fused_experts_w4a16(x, *args)
+    for i in range(3):
+        out.zero_()
+        pkg.fused_experts_w4a16(synth.make_hidden(M, K, dev, seed=70 + i), *args)
+        torch.cuda.synchronize()
+        print(f"xtile replay {i} K={K} N={N}", flush=True)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16)), f"replay {i}"
+    del g
+    pkg.release_graph_workspaces()
