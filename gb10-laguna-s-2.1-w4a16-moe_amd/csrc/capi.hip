@@ -145,32 +145,13 @@ int small_row_tiles(int64_t n_blocks, int64_t rows) {
   return best;
 }
 // Height of the exact-weight tiles (xtile.hip) by average pairs per expert:
-// 32 slots below 24 pairs (the kernel of short tiles has registers for a
-// second set of activation rows: E=256, K=3072, N=1024, 10 pairs per expert
-// 288 us per call against 295, 30 pairs 460 against 404), else 64 (80 pairs
-// per expert at N=128: w13 80 us against 90 with 48-slot tiles), or 48 for groups of 128, whose
+// 32 slots below 24 pairs (the kernel of short tiles holds a second set of
+// activation rows and fragments in registers: E=256, K=3072, N=1024, 10 pairs
+// per expert, w13 192 us against 224), else 64 (80 pairs per expert at N=128:
+// 80 us against 90 with 48-slot tiles), or 48 for groups of 128, whose
 // fragments of a whole group do not fit the registers of taller tiles.
 constexpr int64_t kXTile32MaxPairs = 24;
 constexpr int kXTile128 = 48;
-// Whether the sort and the exact-weight tiles beat the self-routed GEMV: from
-// 2.5 pairs per expert on average, by the two's estimated times.  The GEMV
-// reads an expert's weights once per pass of four pairs, at about 2.4 TB/s
-// with passes that follow one another; the tiles read them once, at 4.2 TB/s,
-// but no faster than 1.05 us per step of 128 elements of a workgroup (w13's
-// reduction, then w2's), and the sort and two launches more take 12 us.
-// Uniform routing, GEMV against tiles: E=64, top-8, K=2048, N=768 M=20 55 / 55
-// us, M=24 65 / 56; E=16, top-4, N=1024 M=16 40 / 43, M=24 52 / 43; E=8,
-// top-2, K=4096, N=1344 M=16 59 / 66, M=24 85 / 66; E=32, top-4, K=1024,
-// N=512 M=24 26 / 31; E=8, top-8, K=4096, N=1024 M=8 50 / 57, M=10 66 / 57.
-// Skewed routing favours the tiles (E=64 M=24 84 / 43).  The margin of 15 %
-// keeps the GEMV where every expert's passes are full.
-bool many_pairs(int64_t n_tok, int64_t E, int64_t N, int64_t K, int64_t group) {
-  if (2 * n_tok < 5 * E) return false;
-  const double mbytes = 3e-6 * (double)(E * N * K) * (0.5 + 2.0 / (double)group);
-  const double passes = (double)n_tok / (4.0 * (double)E) + 0.6;
-  const double steps = (double)((K + 127) / 128 + (N + 127) / 128);
-  return 6.0 + passes * mbytes / 2.4 > 1.15 * (18.0 + std::max(1.05 * steps, mbytes / 4.2));
-}
 constexpr int64_t kXTileMinPairs = 2;  // average pairs per expert they start at
 // Row tiles (`rows` outputs each) one workgroup of the exact-weight tiles runs
 // in turn: about 32 steps of 128 elements, so that short reductions do not
@@ -261,10 +242,8 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
   // every expert goes to the MFMA kernels and the GEMV launches are skipped.
   if (L->mfma && T.auto_split && (int64_t)n_tok >= kAllMfmaMinPairs * E) L->gemv_max_tokens = 0;
   // Small batches: the GEMV kernels route themselves from topk_ids (work
-  // item = one routed expert), so the align kernel is not run -- but not once
-  // their experts hold many pairs, whose passes of four add up.
+  // item = one routed expert), so the align kernel is not run.
   L->route = !L->mfma && M >= 1 && M <= T.gemv_only_max_m &&
-             !(M > T.w2_fused_max_m && many_pairs((int64_t)n_tok, E, N, K, group)) &&
              gemv_route_fits((int)n_tok, (int)E, (int)K, (int)N);
   // Every other call that keeps all experts on exact weights (K or N no
   // multiple of 256, scales that are not 16-byte aligned, or by the tuning):

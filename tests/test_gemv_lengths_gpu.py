@@ -34,23 +34,3 @@ def test_run_time_lengths(pkg, orc, synth, dev, K, N, M):
     # more) times its ulp: the bound of test_fused_sweep_gpu.py, ~2e-3 of
     # max|out| at a weight of one; few rows, so a flip shows in many of them.
     _check(orc, out, x, w13, w2, s13, s2, tw, ti, 32, tag, mismatch_max=0.05, excess_max=2e-3)
-
-
-@pytest.mark.parametrize("E,topk,K,N,M,sorts", [(64, 8, 2048, 768, 19, 0),
-                                                (64, 8, 2048, 768, 20, 1),
-                                                (8, 8, 4096, 1024, 8, 0),
-                                                (8, 8, 4096, 1024, 10, 1),
-                                                (16, 4, 2048, 1024, 24, 1),
-                                                (32, 8, 2048, 512, 10, 0),
-                                                (8, 8, 4096, 1024, 5, 0)])
-def test_many_pairs_take_the_tiles(pkg, orc, synth, dev, E, topk, K, N, M, sorts):
-    """Few-token calls on both sides of the rule that sends them to the sort and
-    the exact-weight tiles; no weight is rounded on either."""
-    tag = f"many pairs E={E} topk={topk} K={K} N={N} M={M}"
-    shape = synth.LayerShape(E=E, topk=topk, K=K, N=N, group=32)
-    assert pkg._lib.stage_launches(M, topk, E, N, K, 32, None)[0] == sorts
-    print(tag, flush=True)
-    w13, w2, s13, s2, x, tw, ti = _make(synth, shape, M, dev, seed=M)
-    out = pkg.fused_experts_w4a16(x, w13, w2, s13, s2, tw, ti, 32)
-    torch.cuda.synchronize()
-    _check(orc, out, x, w13, w2, s13, s2, tw, ti, 32, tag, mismatch_max=0.05, excess_max=2e-3)
