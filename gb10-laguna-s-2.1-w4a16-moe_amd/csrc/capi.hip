@@ -145,10 +145,10 @@ int small_row_tiles(int64_t n_blocks, int64_t rows) {
   return best;
 }
 // Height of the exact-weight tiles (xtile.hip) by average pairs per expert:
-// 32 slots below 24 pairs (the kernel of short tiles holds a second set of
-// activation rows and fragments in registers: E=256, K=3072, N=1024, 10 pairs
-// per expert, w13 192 us against 224), else 64 (80 pairs per expert at N=128:
-// 80 us against 90 with 48-slot tiles), or 48 for groups of 128, whose
+// 32 slots below 24 pairs (the kernel of short tiles has registers for a
+// second set of activation rows: E=256, K=3072, N=1024, 10 pairs per expert
+// 288 us per call against 295, 30 pairs 460 against 404), else 64 (80 pairs
+// per expert at N=128: w13 80 us against 90 with 48-slot tiles), or 48 for groups of 128, whose
 // fragments of a whole group do not fit the registers of taller tiles.
 constexpr int64_t kXTile32MaxPairs = 24;
 constexpr int kXTile128 = 48;
