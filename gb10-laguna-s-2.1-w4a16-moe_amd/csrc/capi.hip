@@ -773,10 +773,17 @@ int w4a16_moe_workspace_size_ex(int64_t M, int64_t topk, int64_t num_experts, in
   Tuning T;
   int st = resolve_tuning(tuning, &T);
   if (st) return st;
-  Layout L;
-  st = compute_layout(M, topk, num_experts, N, K, group_size, T, &L);
-  if (st) return st;
-  *bytes = L.total;
+  // The call's own layout depends on its scales' alignment, which is not known
+  // here: the larger of the two (unaligned scales list sorted blocks where
+  // aligned ones list experts).
+  size_t total = 0;
+  for (const bool scales16 : {true, false}) {
+    Layout L;
+    st = compute_layout(M, topk, num_experts, N, K, group_size, T, &L, scales16);
+    if (st) return st;
+    total = std::max(total, L.total);
+  }
+  *bytes = total;
   return W4A16_OK;
 }
 

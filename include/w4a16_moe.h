@@ -141,7 +141,8 @@ int w4a16_moe_align_block_size_ws(const int32_t* topk_ids, int64_t M,
                                   void* scratch, size_t scratch_bytes, void* stream);
 
 /*
- * Device scratch needed by w4a16_moe_fused_experts (bytes, 256-aligned).
+ * Device scratch needed by w4a16_moe_fused_experts (bytes, 256-aligned), for
+ * scales of any alignment it takes.
  * Replaces the scratch pools _align_workspace / _gemm_workspace,
  * kernels/w4a16_moe.py:141-184 and :293-316.
  */
@@ -149,7 +150,8 @@ int w4a16_moe_workspace_size(int64_t M, int64_t topk, int64_t num_experts,
                              int64_t N, int64_t K, int64_t group_size,
                              size_t* bytes);
 
-/* Byte offsets of the workspace's fields (W4A16_WS_*), for inspection. */
+/* Byte offsets of the workspace's fields (W4A16_WS_*), for inspection, of a
+ * call whose scales are 16-byte aligned. */
 int w4a16_moe_workspace_layout(int64_t M, int64_t topk, int64_t num_experts,
                                int64_t N, int64_t K, int64_t group_size,
                                size_t offsets[W4A16_WS_NFIELDS]);

@@ -136,6 +136,25 @@ def test_fused_validation_codes(lib, pkg):
     assert _fused(lib, M=0, ws_bytes=0) == L.W4A16_OK
 
 
+@pytest.mark.parametrize("thr", [None, 4, 15])
+@pytest.mark.parametrize("M,topk,E,group", [(37, 2, 64, 128), (106, 2, 60, 32), (25, 1, 64, 32),
+                                            (120, 10, 256, 64), (300, 4, 16, 32)])
+def test_workspace_size_covers_unaligned_scales(lib, pkg, M, topk, E, group, thr):
+    """A call whose scales are two bytes off their alignment is laid out
+    without the MFMA split, on both sides of two pairs per expert: a workspace
+    of workspace_size bytes is enough for it.  (The hidden pointer is
+    misaligned, which is checked after the workspace: nothing is launched.)"""
+    L = pkg._lib
+    t = None if thr is None else pkg.Tuning(gemv_only_max_m=0, gemv_max_tokens=thr).to_struct()
+    N, K, P = 256, 512, 1 << 20
+    size = L.workspace_size_ex(M, topk, E, N, K, group, t)
+    tp = None if t is None else ctypes.byref(t)
+    for off in (0, 2):
+        st = lib.w4a16_moe_fused_experts_ex(P + 2, K, P, P, P + off, P + off, P, P, M, topk, E, N,
+                                            K, group, P, K, P, size, None, tp)
+        assert st == L.W4A16_ERR_MISALIGNED, (off, st)
+
+
 def test_align_validation_codes(lib, pkg):
     L = pkg._lib
     P = 1 << 20
