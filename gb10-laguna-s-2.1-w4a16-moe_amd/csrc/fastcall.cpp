@@ -22,6 +22,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <cstdlib>
 #include <tuple>
@@ -325,5 +326,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "w4a16_fastcall", nullptr, -1, meth
 }  // namespace
 
 PyMODINIT_FUNC PyInit_w4a16_fastcall(void) {
-  return PyModule_Create(&module);
+  PyObject* m = PyModule_Create(&module);
+  // checked against the running torch by the loader
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
 }

@@ -4,7 +4,9 @@ Mirrors ``kernels/w4a16_moe.py`` of vladimir-voinea/gb10-laguna-s-2.1-w4a16-moe
 (same function names, positional arguments and argument meaning) on top of the
 HIP library ``libw4a16moe.so`` (C ABI: include/w4a16_moe.h).  PyTorch supplies
 device memory and the current stream only; all arithmetic runs in the HIP
-kernels.  There is no CPU fallback: a missing library raises.
+kernels.  There is no CPU fallback: a missing library raises.  Ordinary calls
+go through native host code (csrc/fastcall.cpp); where that module cannot be
+loaded they run on the path below, with the same results.
 
 Differences from the reference, all deliberate:
   * weights are consumed in the stock pack-quantized layout; ``repack_weights``
@@ -113,7 +115,7 @@ class WorkspacePool:
                 self._on_clear()
 
 
-_WS_POOL = WorkspacePool(on_clear=lambda: _lib.fast().clear_workspaces())
+_WS_POOL = WorkspacePool(on_clear=_lib.clear_native_workspaces)
 
 
 def release_graph_workspaces() -> None:

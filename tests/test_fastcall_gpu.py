@@ -28,6 +28,38 @@ def test_host_tensors_are_left_alone(pkg):
         pkg.fused_experts_w4a16(t, t, t, t, t, t, t)
 
 
+@pytest.fixture(params=["missing", "not loadable"])
+def no_native_module(request, pkg, monkeypatch, tmp_path):
+    """The module cannot be loaded; gives the loaded one."""
+    native = pkg._lib.load_fast()
+    path = tmp_path / "w4a16_fastcall.so"
+    if request.param == "not loadable":
+        path.write_bytes(b"not a library")
+    monkeypatch.setattr(pkg._lib, "FAST_PATH", path)
+    monkeypatch.setattr(pkg._lib, "_fast", None)
+    return native
+
+
+def test_without_the_native_module(pkg, no_native_module, monkeypatch):
+    """The path in Python needs the HIP library only: arguments are checked as
+    ever, and with no library at all too; the pool can be cleared."""
+    pkg.w4a16_moe._WS_POOL.clear()
+    t = torch.zeros(2, 2)
+    with pytest.raises(ImportError):
+        pkg._lib.load_fast()
+    calls = [lambda: pkg.fused_experts_w4a16(t, t, t, t, t, t, t),
+             lambda: pkg.moe_align_block_size(t, 16, 4), lambda: pkg.router_topk_softmax(t, 1)]
+    with pytest.warns(RuntimeWarning, match="native call path"):
+        pkg._lib.fast()
+    for has_library in (True, False):
+        if not has_library:
+            monkeypatch.setattr(pkg._lib, "LIB_PATH", pkg._lib.FAST_PATH.parent / "none.so")
+            monkeypatch.setattr(pkg._lib, "_fast", None)
+        for call in calls:
+            with pytest.raises(pkg._lib.W4A16Error):
+                call()
+
+
 SHAPES = [(16, 4, 512, 256, 32, 6), (16, 4, 512, 256, 64, 40), (8, 2, 96, 160, 32, 90),
           (256, 10, 3072, 1024, 32, 1)]
 
@@ -72,6 +104,24 @@ def test_same_bits_as_the_python_path(pkg, synth, dev, monkeypatch, E, topk, K, 
         pkg.fused_experts_w4a16(x, w13, w2, s13, s2, tw[:, :1], ti, group)
     with torch.device("cuda:0"):  # a torch-function mode
         assert f.fused(*args) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:the native call path")
+def test_same_bits_without_the_native_module(pkg, synth, dev, no_native_module, monkeypatch):
+    shape = synth.LayerShape(E=16, topk=4, K=512, N=256, group=32)
+    w13, w2, s13, s2, x, tw, ti = _make(synth, shape, 6, dev, seed=6)
+    logits = torch.randn((6, 16), device=dev)
+
+    def calls():
+        return [pkg.fused_experts_w4a16(x, w13, w2, s13, s2, tw, ti, 32),
+                *pkg.router_topk_softmax(logits, 4), *pkg.moe_align_block_size(ti, 16, 16)]
+
+    got = calls()
+    assert not isinstance(pkg._lib.fast(), type(no_native_module))
+    monkeypatch.setattr(pkg._lib, "_fast", no_native_module)
+    calls()  # (the native path takes the second call of a shape)
+    assert all(torch.equal(a, b) for a, b in zip(got, calls()))
 
 
 @pytest.mark.gpu
