@@ -51,6 +51,7 @@ WS_NFIELDS = 8
 FUSED_BLOCK_M = 16
 GEMV_MAX_TOKENS = 4
 GEMV_ONLY_MAX_M = 24
+ALIGN_SCRATCH_MIN_PAIRS = 8192
 
 EXPORTED_SYMBOLS = (
     "w4a16_moe_align_sizes",
@@ -177,7 +178,7 @@ class _NoNativePath:
     def _none(self, *args):
         return None
 
-    fused = router = align = set_plan = set_workspace = _none
+    fused = router = align = has_plan = set_plan = set_workspace = _none
     clear_workspaces = clear_plans = _none
 
 

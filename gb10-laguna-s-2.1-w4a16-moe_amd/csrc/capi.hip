@@ -20,6 +20,8 @@ constexpr int64_t kMaxTopk = 256;
 
 size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+static_assert(kAlignChunkedMinPairs == W4A16_ALIGN_SCRATCH_MIN_PAIRS, "as the header says");
+
 int align_sizes(int64_t M, int64_t topk, int64_t E, int64_t block, int64_t* em,
                 int64_t* nb) {
   if (block < 1) return W4A16_ERR_INVALID_BLOCK;

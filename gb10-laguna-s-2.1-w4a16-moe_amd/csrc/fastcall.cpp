@@ -267,6 +267,18 @@ PyObject* py_align(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// has_plan(dev, M, topk, E, N, K, group)
+PyObject* py_has_plan(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  int64_t v[7];
+  if (nargs != 7) {
+    PyErr_SetString(PyExc_TypeError, "has_plan takes 7 integers");
+    return nullptr;
+  }
+  for (int i = 0; i < 7; ++i)
+    if (!as_int(args[i], &v[i])) Py_RETURN_FALSE;
+  return PyBool_FromLong(plans().count(PlanKey{v[0], v[1], v[2], v[3], v[4], v[5], v[6]}) != 0);
+}
+
 // set_plan(dev, M, topk, E, N, K, group, ws_bytes, tuning fields or None)
 PyObject* py_set_plan(PyObject*, PyObject* args) {
   long long dev, M, topk, E, N, K, group, bytes;
@@ -314,6 +326,8 @@ PyMethodDef methods[] = {
     {"router", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(py_router)),
      METH_FASTCALL, nullptr},
     {"align", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(py_align)),
+     METH_FASTCALL, nullptr},
+    {"has_plan", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(py_has_plan)),
      METH_FASTCALL, nullptr},
     {"set_plan", py_set_plan, METH_VARARGS, nullptr},
     {"set_workspace", py_set_workspace, METH_VARARGS, nullptr},

@@ -63,13 +63,16 @@ class WorkspacePool:
     the life of the process.
     """
 
-    def __init__(self, alloc=None, on_clear=None):
+    def __init__(self, alloc=None, on_eager=None, on_clear=None):
+        """on_eager(device, stream, buffer): called with each new eager buffer,
+        on_clear() when every buffer is dropped, both under the pool's lock."""
         self._alloc = alloc or (lambda nbytes, device: torch.empty(
             nbytes, dtype=torch.uint8, device=device))
+        self._on_eager = on_eager
         self._bufs: dict[tuple, torch.Tensor] = {}
         self._retired: list[torch.Tensor] = []  # capture buffers outgrown in their capture
         self._lock = threading.Lock()
-        self._on_clear = on_clear  # called when every buffer is dropped
+        self._on_clear = on_clear
 
     def get(self, device, stream: int, nbytes: int, capture_id: int = 0) -> torch.Tensor:
         """A workspace of at least `nbytes` for a call on `stream`, under the
@@ -83,6 +86,8 @@ class WorkspacePool:
                     self._retired.append(buf)
                 buf = self._alloc(need, device)
                 self._bufs[key] = buf
+                if self._on_eager is not None and not capture_id:
+                    self._on_eager(device, stream, buf)
             return buf
 
     def cached_bytes(self) -> int:
@@ -115,7 +120,13 @@ class WorkspacePool:
                 self._on_clear()
 
 
-_WS_POOL = WorkspacePool(on_clear=_lib.clear_native_workspaces)
+def _show_native(device: torch.device, stream: int, buf: torch.Tensor) -> None:
+    """Give the native call path the eager buffer it is to use from now on."""
+    if device.index is not None:
+        _lib.fast().set_workspace(device.index, stream, buf)
+
+
+_WS_POOL = WorkspacePool(on_eager=_show_native, on_clear=_lib.clear_native_workspaces)
 
 
 def release_graph_workspaces() -> None:
@@ -190,7 +201,9 @@ def _align(topk_ids: torch.Tensor, block_size: int, num_experts: int, with_offse
         dropped = torch.empty(1, dtype=torch.int32, device=dev)
     # Scratch of the many-workgroup sort of large batches (M=4096, top-10:
     # 49.6 us on one workgroup with the router step, 29.1 with it); freed in stream order.
-    nbytes = _lib.align_scratch_size(M, topk, num_experts)
+    nbytes = 0
+    if M * topk >= _lib.ALIGN_SCRATCH_MIN_PAIRS:
+        nbytes = _lib.align_scratch_size(M, topk, num_experts)
     scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
     with torch.cuda.device(dev):
         st = _lib.lib().w4a16_moe_align_block_size_ws(
@@ -243,29 +256,24 @@ def _packed_cols(w: torch.Tensor) -> int:
     return 0
 
 
-def _workspace(device: torch.device, M: int, topk: int, E: int, N: int, K: int,
-               group: int, tuning: "_tuning.Tuning | None" = None) -> torch.Tensor:
-    """The pool's workspace for the current stream, at least this call's size."""
-    ts = None if tuning is None else tuning.to_struct()
+def _workspace(device: torch.device, stream: int, M: int, topk: int, E: int, N: int, K: int,
+               group: int, ts: "_lib.TuningStruct | None" = None) -> torch.Tensor:
+    """The pool's workspace for `stream`, at least this call's size."""
     nbytes = _lib.workspace_size_ex(M, topk, E, N, K, group, ts)
-    stream = _stream_ptr(device)
     cap = _lib.capture_id(stream) if torch.cuda.is_current_stream_capturing() else 0
-    ws = _WS_POOL.get(device, stream, nbytes, capture_id=cap)
-    if not cap and device.index is not None:  # the native call path's view of the pool
-        _lib.fast().set_workspace(device.index, stream, ws)
-    return ws
+    return _WS_POOL.get(device, stream, nbytes, capture_id=cap)
 
 
-def _register_plan(p: "_Prepared") -> None:
-    """Tell the native call path (csrc/fastcall.cpp) how a call of this shape
-    runs when the caller passes no tuning.  It does not take calls while a
-    tuning environment variable is set, so none may enter here."""
-    if p.device.index is None or any(os.environ.get(v) for v in _TUNING_ENV):
+def _register_plan(p: "_Prepared", ts: "_lib.TuningStruct | None") -> None:
+    """Tell the native call path (csrc/fastcall.cpp), once, how a call of this
+    shape runs when the caller passes no tuning.  It does not take calls while
+    a tuning environment variable is set, so none may enter here."""
+    key = (p.device.index, p.M, p.topk, p.E, p.N, p.K, p.group)
+    fast = _lib.fast()
+    if key[0] is None or fast.has_plan(*key) or any(os.environ.get(v) for v in _TUNING_ENV):
         return
-    ts = None if p.tuning is None else p.tuning.to_struct()
-    nbytes = _lib.workspace_size_ex(p.M, p.topk, p.E, p.N, p.K, p.group, ts)
     fields = None if ts is None else tuple(int(getattr(ts, f)) for f, _ in ts._fields_)
-    _lib.fast().set_plan(p.device.index, p.M, p.topk, p.E, p.N, p.K, p.group, nbytes, fields)
+    fast.set_plan(*key, _lib.workspace_size_ex(*key[1:], ts), fields)
 
 
 class _Prepared:
@@ -339,16 +347,15 @@ def _tuning_for(p: _Prepared, tuning) -> None:
     p.tuning = tuning
 
 
-def _tuning_ptr(p: _Prepared):
-    return None if p.tuning is None else ctypes.byref(p.tuning.to_struct())
+def _tuning_struct(tuning: "_tuning.Tuning | None") -> "_lib.TuningStruct | None":
+    return None if tuning is None else tuning.to_struct()
 
 
-def _fused_args(p: _Prepared, out: torch.Tensor, ws: torch.Tensor):
+def _fused_args(p: _Prepared, out: torch.Tensor, ws: torch.Tensor, stream: int):
     return (p.hidden.data_ptr(), p.hidden.stride(0), p.w1_q.data_ptr(), p.w2_q.data_ptr(),
             p.w1_scale.data_ptr(), p.w2_scale.data_ptr(), p.topk_weights.data_ptr(),
             p.topk_ids.data_ptr(), p.M, p.topk, p.E, p.N, p.K, p.group,
-            out.data_ptr(), out.stride(0), ws.data_ptr(), ws.numel(),
-            _stream_ptr(p.device))
+            out.data_ptr(), out.stride(0), ws.data_ptr(), ws.numel(), stream)
 
 
 def fused_experts_w4a16(
@@ -401,12 +408,15 @@ def fused_experts_w4a16(
     if p.M == 0:
         return out
     _tuning_for(p, tuning)
-    ws = _workspace(p.device, p.M, p.topk, p.E, p.N, p.K, p.group, p.tuning)
+    ts = _tuning_struct(p.tuning)
+    stream = _stream_ptr(p.device)
+    ws = _workspace(p.device, stream, p.M, p.topk, p.E, p.N, p.K, p.group, ts)
     with torch.cuda.device(p.device):
-        st = _lib.lib().w4a16_moe_fused_experts_ex(*_fused_args(p, out, ws), _tuning_ptr(p))
+        st = _lib.lib().w4a16_moe_fused_experts_ex(
+            *_fused_args(p, out, ws, stream), None if ts is None else ctypes.byref(ts))
     _lib.check(st)
     if tuning is None:
-        _register_plan(p)
+        _register_plan(p, ts)
     return out
 
 
@@ -423,9 +433,10 @@ def fused_experts_w4a16_profiled(hidden, w1_q, w2_q, w1_scale, w2_scale, topk_we
     ms = (ctypes.c_float * 4)()
     if p.M == 0:
         return out, dict.fromkeys(("align", "w13", "w2", "combine"), 0.0)
-    ws = _workspace(p.device, p.M, p.topk, p.E, p.N, p.K, p.group)
+    stream = _stream_ptr(p.device)
+    ws = _workspace(p.device, stream, p.M, p.topk, p.E, p.N, p.K, p.group)
     with torch.cuda.device(p.device):
-        st = _lib.lib().w4a16_moe_fused_experts_profiled(*_fused_args(p, out, ws), ms)
+        st = _lib.lib().w4a16_moe_fused_experts_profiled(*_fused_args(p, out, ws, stream), ms)
     _lib.check(st)
     return out, {"align": ms[0], "w13": ms[1], "w2": ms[2], "combine": ms[3]}
 
@@ -442,8 +453,8 @@ def workspace_tensor(hidden: torch.Tensor, topk_ids: torch.Tensor, w1_q: torch.T
     N = w1_q.shape[1] // 2
     if tuning is None:
         tuning = _tuning.select(M, E, N, K, group_size, hidden.device)
-    ws = _workspace(hidden.device, M, topk, E, N, K, group_size, tuning)
-    ts = None if tuning is None else tuning.to_struct()
+    ts = _tuning_struct(tuning)
+    ws = _workspace(hidden.device, _stream_ptr(hidden.device), M, topk, E, N, K, group_size, ts)
     return ws, _lib.workspace_layout_ex(M, topk, E, N, K, group_size, ts)
 
 

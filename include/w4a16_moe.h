@@ -123,11 +123,14 @@ int w4a16_moe_align_block_size(const int32_t* topk_ids, int64_t M,
                                int32_t* expert_offsets, int32_t* dropped,
                                void* stream);
 
+/* Pairs from which the sort below may use scratch. */
+#define W4A16_ALIGN_SCRATCH_MIN_PAIRS 8192
+
 /*
  * The same with device scratch of w4a16_moe_align_scratch_size bytes (4-byte
- * aligned; 0 bytes: none is used and `scratch` may be NULL): batches of 8,192
- * pairs or more (E <= 512) then sort on one workgroup per 1,024 pairs, in two
- * launches.  Same outputs, bit for bit.  The scratch need not be cleared and
+ * aligned; 0 bytes: none is used and `scratch` may be NULL): batches of
+ * W4A16_ALIGN_SCRATCH_MIN_PAIRS pairs or more (E <= 512) then sort on one
+ * workgroup per 1,024 pairs, in two launches.  Same outputs, bit for bit.  The scratch need not be cleared and
  * is free for other work after the call in stream order.
  */
 int w4a16_moe_align_scratch_size(int64_t M, int64_t topk, int64_t num_experts,

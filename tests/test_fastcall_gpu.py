@@ -37,7 +37,8 @@ def no_native_module(request, pkg, monkeypatch, tmp_path):
         path.write_bytes(b"not a library")
     monkeypatch.setattr(pkg._lib, "FAST_PATH", path)
     monkeypatch.setattr(pkg._lib, "_fast", None)
-    return native
+    yield native
+    pkg.w4a16_moe._WS_POOL.clear()  # the next buffers are shown to the module again
 
 
 def test_without_the_native_module(pkg, no_native_module, monkeypatch):
@@ -122,6 +123,71 @@ def test_same_bits_without_the_native_module(pkg, synth, dev, no_native_module, 
     monkeypatch.setattr(pkg._lib, "_fast", no_native_module)
     calls()  # (the native path takes the second call of a shape)
     assert all(torch.equal(a, b) for a, b in zip(got, calls()))
+
+
+class _Counting:
+    """The native module, counting what is registered."""
+
+    def __init__(self, native):
+        self.native, self.seen = native, []
+
+    def __getattr__(self, name):
+        if name.startswith("set_"):
+            self.seen.append(name)
+        return getattr(self.native, name)
+
+
+def test_each_eager_buffer_is_shown_once(pkg):
+    """Threads on one stream whose calls grow its buffer: what the pool shows
+    last is what it holds, and nothing is shown for a buffer that is reused
+    or belongs to a capture."""
+    shown = {}
+    count = [0]
+
+    def on_eager(device, stream, buf):
+        shown[stream] = buf
+        count[0] += 1
+
+    pool = pkg.w4a16_moe.WorkspacePool(
+        alloc=lambda n, d: torch.empty(n, dtype=torch.uint8), on_eager=on_eager,
+        on_clear=shown.clear)
+    sizes = [400 + 7 * i for i in range(200)]
+
+    def worker(k):
+        for n in sizes[k::4]:
+            pool.get("cuda:0", 5, n)
+            pool.get("cuda:0", 5, 300)
+            pool.get("cuda:0", 5, n, capture_id=9)
+
+    threads = [threading.Thread(target=worker, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert shown[5] is pool.get("cuda:0", 5, 1) and shown[5].numel() == max(sizes)
+    assert count[0] <= len(sizes)
+    pool.clear()
+    assert not shown
+
+
+@pytest.mark.gpu
+def test_declined_calls_register_nothing_again(pkg, synth, dev, monkeypatch):
+    shape = synth.LayerShape(E=16, topk=4, K=512, N=256, group=32)
+    w13, w2, s13, s2, x, tw, ti = _make(synth, shape, 6, dev, seed=8)
+    odd = torch.zeros(6, 516, dtype=torch.bfloat16, device=dev)[:, :512]
+    odd.copy_(x)
+    native = pkg._lib.load_fast()
+    native.clear_plans()
+    pkg.w4a16_moe._WS_POOL.clear()
+    counting = _Counting(native)
+    monkeypatch.setattr(pkg._lib, "_fast", counting)
+    t = pkg.Tuning()
+    for i in range(3):  # declined for its row stride, and for its tuning
+        a = pkg.fused_experts_w4a16(odd, w13, w2, s13, s2, tw, ti, 32)
+        b = pkg.fused_experts_w4a16(x, w13, w2, s13, s2, tw, ti, 32, tuning=t)
+        assert sorted(counting.seen) == ["set_plan", "set_workspace"], i
+    assert torch.equal(_bits(native.fused(x, w13, w2, s13, s2, tw, ti, 32)), _bits(a))
+    assert torch.equal(_bits(a), _bits(b))
 
 
 @pytest.mark.gpu
