@@ -229,6 +229,12 @@ def clear_native_workspaces() -> None:
         _fast.clear_workspaces()
 
 
+def clear_native_plans() -> None:
+    """Drop the native call path's dispatch choices, if it is loaded."""
+    if _fast is not None:
+        _fast.clear_plans()
+
+
 def strerror(status: int) -> str:
     return lib().w4a16_moe_strerror(status).decode()
 

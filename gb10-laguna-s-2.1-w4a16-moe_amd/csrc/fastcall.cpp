@@ -8,9 +8,10 @@
 // always did.  A one-token call spent 27 us in Python for 15 us of kernels.
 //
 // Plans (dispatch choices and workspace bytes by shape) and workspaces (by
-// device and stream) are the Python layer's: it registers them here after its
-// own path has made them, and clears them here when it drops its own.  All
-// state is read and written with the GIL held.
+// device and stream) come from the Python layer: it registers a plan after its
+// own path has run the shape once (kept until tuning.reload_tables()), shows
+// every eager buffer its pool makes, and clears them here when the pool drops
+// its own.  All state is read and written with the GIL held.
 #include <Python.h>
 
 #include <ATen/ATen.h>

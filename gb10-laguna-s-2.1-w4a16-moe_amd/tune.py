@@ -271,6 +271,7 @@ def main(argv=None) -> int:
         old = T.load_table(args.E, args.N, args.K, args.group, T.device_name(), out_dir) or {}
         table = {**{m: t for m, t in old.items() if m not in table}, **table}
     path.write_text(T.dump_table(table))
+    T.reload_tables()
     log(f"wrote {path}")
     if args.report:
         Path(args.report).write_text(json.dumps({"device": T.device_name(), "E": args.E,

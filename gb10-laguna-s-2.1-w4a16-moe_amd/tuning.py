@@ -12,6 +12,9 @@ kernels' tile shapes themselves are fixed at build time.
 Files live in ``configs/`` next to this module (or in $W4A16_MOE_CONFIG_DIR)
 and are written by ``tune.py``.  Without a file for the shape and device the
 library's built-in choices apply.  W4A16_MOE_TUNING=default ignores the files.
+A file is read once per process, and the native call path keeps the choice made
+for a shape: a program that rewrites a file, or points CONFIG_DIR elsewhere,
+calls ``reload_tables()``.
 """
 
 from __future__ import annotations
@@ -25,7 +28,8 @@ from pathlib import Path
 from . import _lib
 
 CONFIG_DIR = Path(__file__).resolve().parent / "configs"
-# gemv_only_max_m that means "every M in this bucket runs GEMV-only"
+# gemv_only_max_m that means "every M in this bucket keeps all experts on exact
+# weights": the GEMV, or the exact-weight tiles of calls with many pairs
 ALWAYS = 1 << 30
 
 
@@ -115,6 +119,12 @@ def _load(path: str) -> dict[int, Tuning] | None:
     if not p.exists():
         return None
     return parse_table(p.read_text())
+
+
+def reload_tables() -> None:
+    """Forget the tables read so far and the dispatch choices made from them."""
+    _load.cache_clear()
+    _lib.clear_native_plans()
 
 
 def load_table(E: int, N: int, K: int, group: int, dev_name: str,

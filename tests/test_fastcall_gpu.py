@@ -125,6 +125,42 @@ def test_same_bits_without_the_native_module(pkg, synth, dev, no_native_module, 
     assert all(torch.equal(a, b) for a, b in zip(got, calls()))
 
 
+def _table(pkg, folder, tuning):
+    T = pkg.tuning
+    (folder / T.config_name(16, 256, 512, 32, T.device_name() if torch.cuda.is_available()
+                            else "dev")).write_text(T.dump_table({8: tuning}))
+
+
+def test_reload_tables(pkg, tmp_path):
+    T = pkg.tuning
+    a, b = T.Tuning(T.ALWAYS, 4, 2, 0), T.Tuning(0, 0, 0, 0)
+    for want in (a, b):
+        _table(pkg, tmp_path, want)
+        T.reload_tables()
+        name = T.device_name() if torch.cuda.is_available() else "dev"
+        assert T.load_table(16, 256, 512, 32, name, tmp_path) == {8: want}
+
+
+@pytest.mark.gpu
+def test_reload_tables_reaches_the_native_path(pkg, synth, dev, tmp_path, monkeypatch):
+    """A rewritten table decides the next call's dispatch (tiles in header[2])."""
+    T = pkg.tuning
+    shape = synth.LayerShape(E=16, topk=4, K=512, N=256, group=32)
+    w13, w2, s13, s2, x, tw, ti = _make(synth, shape, 40, dev, seed=5)
+    args = (x, w13, w2, s13, s2, tw, ti, 32)
+    monkeypatch.setattr(T, "CONFIG_DIR", tmp_path)
+    tiles = []
+    for tuning in (T.Tuning(0, 15, 0, 64), T.Tuning(0, 0, 0, 64)):
+        _table(pkg, tmp_path, tuning)
+        T.reload_tables()
+        pkg.fused_experts_w4a16(*args)
+        assert pkg._lib.fast().fused(*args) is not None
+        ws, off = pkg.workspace_tensor(x, ti, w13, w2, 32)
+        tiles.append(int(ws[off[2] + 8: off[2] + 12].view(torch.int32).item()))
+    T.reload_tables()
+    assert tiles[0] < tiles[1] == int(torch.unique(ti).numel())
+
+
 class _Counting:
     """The native module, counting what is registered."""
 
