@@ -137,8 +137,16 @@ struct AlignLaunch {
 };
 constexpr int kAlignChunkedMinPairs = 8192;
 constexpr int kAlignChunkedMaxE = 512;
+// Every workgroup of the many-workgroup sort reads the counts of all chunks,
+// so it grows with the square of the batch where one workgroup grows with the
+// batch: pairs x experts up to which it is the faster one (E=512, 4.2, 6.3 and
+// 8.4 million pairs 2.7, 5.6 and 9.8 ms against 4.1, 6.2 and 8.3; E=256, 12.6
+// and 16.8 million 10.9 and 19.3 against 11.7 and 15.6; E=64, 50 and 67
+// million 43 and 76 against 47 and 69).
+constexpr int64_t kAlignChunkedMaxWork = (int64_t)3 << 30;
 inline bool align_is_chunked(int64_t n_tok, int64_t num_experts) {
-  return n_tok >= kAlignChunkedMinPairs && num_experts <= kAlignChunkedMaxE;
+  return n_tok >= kAlignChunkedMinPairs && num_experts <= kAlignChunkedMaxE &&
+         n_tok * num_experts <= kAlignChunkedMaxWork;
 }
 int align_chunks(int n_tok);
 inline size_t align_chunk_scratch_ints(int n_tok, int num_experts) {

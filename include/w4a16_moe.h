@@ -129,8 +129,8 @@ int w4a16_moe_align_block_size(const int32_t* topk_ids, int64_t M,
 /*
  * The same with device scratch of w4a16_moe_align_scratch_size bytes (4-byte
  * aligned; 0 bytes: none is used and `scratch` may be NULL): batches of
- * W4A16_ALIGN_SCRATCH_MIN_PAIRS pairs or more (E <= 512) then sort on one
- * workgroup per 1,024 pairs, in two launches.  Same outputs, bit for bit.  The scratch need not be cleared and
+ * W4A16_ALIGN_SCRATCH_MIN_PAIRS pairs or more (E <= 512, pairs x E at most
+ * 3 * 2^30) then sort on one workgroup per 1,024 pairs, in two launches.  Same outputs, bit for bit.  The scratch need not be cleared and
  * is free for other work after the call in stream order.
  */
 int w4a16_moe_align_scratch_size(int64_t M, int64_t topk, int64_t num_experts,

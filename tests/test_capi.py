@@ -165,6 +165,17 @@ def test_align_validation_codes(lib, pkg):
     assert f(P, 4, 0, 8, 16, P, P, P, None, None, None) == L.W4A16_ERR_INVALID_SHAPE
 
 
+@pytest.mark.parametrize("E", [64, 256, 512])
+def test_many_workgroup_sort_limits(pkg, E):
+    """The sort over many workgroups runs from 8,192 pairs to 3 * 2^30 pairs x
+    experts, standalone and inside the fused call."""
+    L = pkg._lib
+    top = (3 << 30) // E
+    for pairs, many in ((8191, False), (8192, True), (top, True), (top + 1, False)):
+        assert (L.align_scratch_size(pairs, 1, E) > 0) == many
+        assert L.stage_launches(pairs, 1, E, 32, 32, 32, None)[0] == (2 if many else 1)
+
+
 def test_null_output_pointers(lib, pkg):
     L = pkg._lib
     assert lib.w4a16_moe_workspace_size(1, 1, 1, 32, 32, 32, None) == L.W4A16_ERR_NULL_POINTER
