@@ -103,7 +103,8 @@ __device__ void block_exclusive_scan_n(const int (&v)[NV], int (&excl)[NV], int 
 // Token blocks of the tallest tile (MFMA tiles: 32 slots a block; exact-weight
 // tiles: 16): the tile list is ordered by height class, tallest first.
 constexpr int kTileClasses = kMfmaTileMMax / 32;
-static_assert(kXTileM / 16 <= kTileClasses, "height classes of the exact-weight tiles");
+// The exact-weight tiles have fewer classes: the two tallest carry few_pairs.
+static_assert(kXTileM / 16 <= kTileClasses - 2, "height classes of the exact-weight tiles");
 __device__ __forceinline__ int block_shift(const AlignLaunch& a) { return a.xtiles ? 4 : 5; }
 
 // Work lists of the fused call.  An expert with more than gemv_max_tokens
@@ -165,6 +166,7 @@ __device__ void scan_inputs(const AlignLaunch& a, const int32_t* tot, int e0, in
       const int kf = cls(per), kl = cls(c - (n_t - 1) * per);
 #pragma unroll
       for (int k = 0; k < NC; ++k) v[k] += (k == kf ? n_t - 1 : 0) + (k == kl ? 1 : 0);
+      if (a.xtiles) v[0] += few_pairs_cost(c), v[1] += few_pairs_over(c);
     } else if (c > 0) {
       ++v[NC];
     }
@@ -182,7 +184,7 @@ __device__ void write_work_lists(const AlignLaunch& a, const int32_t* tot, const
 #pragma unroll
   for (int k = 0; k < NC; ++k) {
     pos[k] = excl[k] + n_tiles;
-    n_tiles += total[k];
+    if (k >= 2 || !a.xtiles) n_tiles += total[k];
   }
   pos[NC] = excl[NC];
   for (int i = 0; i < ipt; ++i) {
@@ -210,7 +212,8 @@ __device__ void write_work_lists(const AlignLaunch& a, const int32_t* tot, const
   }
   if (scalars) {
     a.n_tiles[0] = n_tiles;
-    if (a.n_gemv) a.n_gemv[0] = total[NC];
+    a.n_gemv[0] = total[NC];  // (exact-weight tiles: none)
+    if (a.xtiles) a.few_pairs[0] = total[0], a.few_pairs[1] = total[1];
   }
 }
 

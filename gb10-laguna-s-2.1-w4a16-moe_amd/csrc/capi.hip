@@ -258,7 +258,10 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
   // N=320: M=25 38.9 against 43.3 us, M=48 50.5 against 57.6, M=64 60.8
   // against 57.6; E=256, top-10, K=3072, N=128: M=25 60.5 against 64.6, M=39
   // 80.5 against 70.3).  Under skewed routing the tiles win everywhere (M=25
-  // 57 against 39 us), but the host does not see the routing.
+  // 57 against 39 us), but the host does not see the routing.  Nor does it see
+  // how many pairs belong to experts elsewhere: the tiles' launches look at
+  // the sort's counts and run the GEMV's items where few are left
+  // (few_pairs_gemv in xtile.hip).
   L->xtile = !L->mfma && !L->route && (int64_t)n_tok >= kXTileMinPairs * E;
   L->gemv = L->mfma ? L->gemv_max_tokens > 0 : !L->xtile;
   L->tc = T.tc;
@@ -557,6 +560,8 @@ int run_fused(const FusedArgs& a, const Layout& L, hipStream_t stream, hipEvent_
   if (L.xtile) {
     al.xtiles = reinterpret_cast<int32_t*>(w.tiles);
     al.n_tiles = w.header + 2;
+    al.n_gemv = w.header + 3;
+    al.few_pairs = w.header + 4;
     al.tile_m = L.xtile_m;
   } else if (L.mfma) {
     al.tiles = w.tiles;

@@ -125,6 +125,7 @@ struct AlignLaunch {
   // Requires gemv_max_tokens < block.
   int4* tiles;           // [max tiles] (expert, first slot, count, 0)
   int32_t* xtiles;       // exact-weight tiles instead: first slot / 16 | blocks of 16 << 28
+  int32_t* few_pairs;    // with xtiles: [2] sums of few_pairs_cost and few_pairs_over
   int32_t* n_tiles;      // [1]
   int32_t* gemv_blocks;  // [max blocks] block indices, ascending
   int32_t* n_gemv;       // [1]
@@ -211,7 +212,7 @@ struct MfmaLaunch {
   const uint16_t* s;       // bf16 scales   [E, rows_total, kdim/G]
   const int32_t* sorted;
   const int4* tiles;       // (expert, first slot, count, 0)
-  const int32_t* header;   // [2] = number of tiles
+  const int32_t* header;   // [0] = padded slots, [2] = number of tiles, [4], [5] = few_pairs
   const float* topk_w;     // w2 only
   void* out;               // w13: bf16 inter [n_tok, n_out]; w2: partial [n_tok, n_out]
   int32_t partial_bf16;    // w2: partial rows are bf16 (else fp32)
@@ -220,6 +221,7 @@ struct MfmaLaunch {
   int32_t n_out;           // N for w13 (2N weight rows), K for w2
   int32_t kdim;
   int32_t group;
+  int32_t few_cost[2];     // set by the launcher (few_pairs_gemv in xtile.hip)
   int32_t max_tiles;
   int32_t tile_m;          // token slots per tile, at most (128 or 192)
   int32_t row_tiles;       // row tiles (of the geometry's height) one workgroup runs in turn
@@ -230,6 +232,19 @@ hipError_t launch_w2_mfma(const MfmaLaunch& a, hipStream_t stream);
 // Exact-weight tiles (xtile.hip): an expert's pairs are cut into tiles of at
 // most kXTileM slots.
 constexpr int kXTileM = 64;
+// What the sort tells them about the experts' pair counts, so that a call that
+// the host took for a large one, but most of whose pairs belong to experts
+// elsewhere, can run the GEMV's items instead (few_pairs_gemv in xtile.hip).
+// An expert's share of the GEMV's time, in units of half a one-row pass (240
+// experts of N=1056, K=3072: 147, 225 and 423 us for 1, 4 and 8 pairs each):
+__host__ __device__ constexpr int few_pairs_cost(int pairs) {
+  return pairs == 0 ? 0 : pairs <= 2 ? 2 : pairs <= 4 ? 3 : 6;
+}
+// and whether it takes more than one pass (> 4 pairs) or two (kFewPairsOver).
+constexpr int kFewPairsOver = 2048;  // more than the count of single ones, 1,024
+__host__ __device__ constexpr int few_pairs_over(int pairs) {
+  return pairs > 8 ? kFewPairsOver : pairs > 4 ? 1 : 0;
+}
 struct XtileLaunch {
   const uint16_t* act;     // bf16 activation rows (x for w13, inter for w2)
   int64_t ld_act;
@@ -238,7 +253,7 @@ struct XtileLaunch {
   const int32_t* sorted;
   const int32_t* expert_ids;
   const int32_t* tiles;    // first slot / 16 | blocks of 16 slots << 28
-  const int32_t* header;   // [2] = number of tiles
+  const int32_t* header;   // [0] = padded slots, [2] = number of tiles, [4], [5] = few_pairs
   const float* topk_w;     // w2 only
   void* out;               // w13: bf16 inter [n_tok, n_out]; w2: partial [n_tok, n_out]
   int32_t partial_bf16;    // w2: partial rows are bf16 (else fp32)
@@ -247,6 +262,7 @@ struct XtileLaunch {
   int32_t n_out;           // N for w13 (2N weight rows), K for w2
   int32_t kdim;
   int32_t group;
+  int32_t few_cost[2];     // set by the launcher (few_pairs_gemv in xtile.hip)
   int32_t max_tiles;
   int32_t tile_m;          // slots per tile, at most (<= kXTileM)
   int32_t row_tiles;       // row tiles (256 weight rows) one workgroup runs in turn

@@ -701,7 +701,7 @@ constexpr size_t kMaxLds = 65536;
 #endif
 constexpr int kGemvWaves = W4A16_GEMV_WAVES;
 
-size_t gemv_lds_bytes(int tc, int kdim) {
+__host__ __device__ __forceinline__ size_t gemv_lds_bytes(int tc, int kdim) {
   const size_t row_oct = (size_t)staged_row_octets(kdim);
   return tc * (row_oct * sizeof(u32x4_t) + (size_t)((kdim >> 5) + 1) * sizeof(float));
 }

@@ -40,10 +40,13 @@
 // waves per SIMD, 440 VALU instructions per wave and step of which 192 are
 // the groups' multiply-adds), with few the memory (10 pairs at N=1024: w13
 // 192 us, 4.7 TB/s of weights).
+#include <limits.h>
+
 #include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
+#include "gemv_item.hpp"
 
 namespace w4a16 {
 namespace {
@@ -57,6 +60,7 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kWaves = 4;
 constexpr int kRB = 4;            // 16-row blocks per wave
 constexpr int kXcds = 8;
+constexpr int kGemvLds = 76 * 1024;
 
 // LDS of one workgroup for tiles of at most TBMAX token blocks: two
 // activation buffers of one step, each wave's packed weights of a pair of
@@ -74,7 +78,8 @@ struct XGeo {
   static constexpr int kS = 64 * kSRow;
   static constexpr int kOffW = 2 * TBMAX * 4096;
   static constexpr int kOffS = kOffW + kWaves * kW;
-  static constexpr int kLds = kOffS + kWaves * kS;
+  // (at least what the GEMV's items stage of rows of up to 7,360 elements)
+  static constexpr int kLds = kOffS + kWaves * kS > kGemvLds ? kOffS + kWaves * kS : kGemvLds;
   static_assert(2 * (kLds + kTileM * 8) <= 160 * 1024, "two workgroups per CU");
 };
 
@@ -529,6 +534,69 @@ __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, 
   }
 }
 
+// ---- calls with few pairs per expert -----------------------------------------
+// The host lays out a call by all its pairs; where most of them belong to
+// experts elsewhere (one GPU's share of the experts), an expert is left with a
+// pair or two and a tile's chain of steps is the launch: 27 us for w13 at
+// K=3072 however few tiles there are, where the GEMV takes 8 to 20.  Such a
+// launch runs the GEMV's items instead, its workgroups taking them in turn,
+// by the counts that the sort left in the header:
+//   cost   few_pairs_cost summed,
+//   over   experts of more than one pass (kFewPairsOver each: of more than two),
+//   experts  routed experts (one sorted block each, as over < kFewPairsOver).
+// w13: while the GEMV is not bound by throughput (few_cost, by what its passes
+// and a tile's steps take: set_few_pairs), or nearly every expert has one or
+// two pairs.  E=32 of 256, K=3072, N=128, 25 and 48 tokens of top-10: w13 27.1
+// -> 10 us, 27.2 -> 18 (the GEMV's own launch 9.8 and 17.0).
+// w2: while no expert takes a second pass (N=1056, K=3072: 20 experts of 1, 4
+// and 8 pairs 13, 17 and 29 us against 28 to 29; 240 of them 123, 151 and 297
+// against 154 to 164) and, for short rows, whose tiles are short too, the
+// items are few.  The branch costs the launches that run their tiles 0 to 0.4
+// us, those of 16-slot tiles with groups of 64 (other registers) 0.7 to 1.
+template <int MODE>
+__device__ __forceinline__ bool few_pairs_gemv(const XtileLaunch& a, int experts, int cost,
+                                               int over) {
+  if (MODE == 1) return over == 0 && cost <= a.few_cost[0];
+  return over < kFewPairsOver && (cost <= a.few_cost[over > 0] ||
+                                  (a.few_cost[0] >= 0 && over == 0 && 4 * cost <= 9 * experts));
+}
+
+// The GEMV's shape: that of its passes of four rows (two where four do not
+// fit the LDS).
+constexpr int gemv_rpl(int mode) { return mode == 0 ? W4A16_W13_RPL_T4 : W4A16_W2_RPL_T4; }
+constexpr int gemv_pf(int mode) { return mode == 0 ? W4A16_W13_PF_T4 : W4A16_W2_PF_T4; }
+__host__ __device__ constexpr int gemv_groups(int mode, int n_out) {
+  return (n_out + 8 * gemv_rpl(mode) * kWaves - 1) / (8 * gemv_rpl(mode) * kWaves);
+}
+
+template <int MODE, int TC>
+__device__ __forceinline__ void run_gemv(const XtileLaunch& a, int experts, unsigned char* lds) {
+  static_assert(gemv_dev::kGemvWaves == kWaves, "workgroups of one size");
+  GemvLaunch g{};
+  g.act = a.act;
+  g.ld_act = a.ld_act;
+  g.w = a.w;
+  g.s = a.s;
+  g.sorted = a.sorted;
+  g.expert_ids = a.expert_ids;
+  g.header = a.header;
+  g.topk_w = a.topk_w;
+  g.out = a.out;
+  g.partial_bf16 = a.partial_bf16;
+  g.n_tok = a.n_tok;
+  g.topk = a.topk;
+  g.n_out = a.n_out;
+  g.kdim = a.kdim;
+  g.block = 16;
+  g.group = a.group;
+  g.nib_mask = a.nib_mask;
+  g.nib_magic = a.nib_magic;
+  const int items = experts * gemv_groups(MODE, a.n_out);
+  for (int i = (int)blockIdx.x; i < items; i += (int)gridDim.x)
+    gemv_dev::gemv_item<MODE, gemv_rpl(MODE), gemv_pf(MODE), TC, kWaves, 0, false, 1, 8>(
+        g, i, reinterpret_cast<gemv_dev::u32x4_t*>(lds));
+}
+
 template <int MODE, int GS, int SP, class X>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void xtile_kernel(const XtileLaunch a) {
@@ -545,6 +613,14 @@ void xtile_kernel(const XtileLaunch a) {
   const int xcd = bid % kXcds, slot = bid / kXcds;
   const int round = slot / items;
   const int tile = kXcds * round + ((round & 1) ? kXcds - 1 - xcd : xcd);
+  const int experts = a.header[0] >> 4;
+  if (few_pairs_gemv<MODE>(a, experts, a.header[4], a.header[5])) {
+    if (MODE == 1 || gemv_dev::gemv_lds_bytes(4, a.kdim) <= kGemvLds)
+      run_gemv<MODE, 4>(a, experts, lds);
+    else
+      run_gemv<MODE, MODE == 0 ? 2 : 4>(a, experts, lds);
+    return;
+  }
   if (tile >= a.header[2]) return;
   const int rt0 = (slot - round * items) * a.row_tiles;
   const int nrt = min(a.row_tiles, n_rt - rt0);
@@ -613,6 +689,32 @@ hipError_t launch_geo(const XtileLaunch& a, dim3 g, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Costs up to which few_pairs_gemv takes the GEMV, for experts of at most one
+// and two passes.  w13: a tile's chain takes about 3.5 + 7.6e-3 K us, the
+// GEMV 0.6 of its own chain (3 + 2.75e-3 K us a pass) and 0.095 us per unit of
+// cost and million weights (N K); fitted to K from 1,024 to 6,144 and N from
+// 96 to 1,408, 4 to 240 experts of 1, 4 and 8 pairs (the sum of a call whose
+// experts mix one and two passes stays lower: 128 of 256 experts, N=128, 64
+// tokens, cost 320, GEMV 59.1 us per call, tiles 57.4).  w2: rows of one step
+// (N <= 128) and of two, by their number of rows (N=128, K=3072: 20 experts
+// of 1 and 4 pairs 5.6 and 7.1 us against 7.2, 48 of them 10.5 and 13.4
+// against 10.3; N=192, K=6144: 48 experts 17.7 and 22.8 against 22.6 and
+// 23.7, 60 of them 22.2 against 18.9); longer rows always.
+template <int MODE>
+void set_few_pairs(XtileLaunch& a) {
+  using gemv_dev::gemv_lds_bytes;
+  const bool four = gemv_lds_bytes(4, a.kdim) <= kGemvLds;
+  a.few_cost[0] = a.few_cost[1] = -1;
+  if (MODE == 0 && gemv_lds_bytes(2, a.kdim) <= kGemvLds) {
+    const int steps = 18000000 / a.kdim;
+    const int one = (62000 + steps) / a.n_out, two = (32000 + steps) / a.n_out;
+    a.few_cost[0] = four ? one : two;  // (two-row passes: twice as many)
+    a.few_cost[1] = four ? two : -1;
+  } else if (MODE == 1 && four) {
+    a.few_cost[0] = a.kdim <= 128 ? 160000 / a.n_out : a.kdim <= 256 ? 600000 / a.n_out : INT_MAX;
+  }
+}
+
 template <int MODE>
 hipError_t launch_xtile(const XtileLaunch& a_in, hipStream_t stream) {
   XtileLaunch a = a_in;
@@ -624,8 +726,12 @@ hipError_t launch_xtile(const XtileLaunch& a_in, hipStream_t stream) {
   const int rows_per_tile = MODE == 0 ? kWaves * 32 : kWaves * 64;
   const int n_rt = (a.n_out + rows_per_tile - 1) / rows_per_tile;
   const int items = (n_rt + a.row_tiles - 1) / a.row_tiles;
-  const int64_t grid = (int64_t)(a.max_tiles + kXcds - 1) / kXcds * kXcds * items;
+  int64_t grid = (int64_t)(a.max_tiles + kXcds - 1) / kXcds * kXcds * items;
   if (grid <= 0) return hipSuccess;
+  set_few_pairs<MODE>(a);
+  if (a.few_cost[0] >= 0)  // enough for the GEMV's items: two workgroups per CU
+    grid = std::max(grid, std::min<int64_t>(512, (int64_t)a.max_tiles *
+                                                     gemv_groups(MODE, a.n_out)));
   if (grid > INT32_MAX) return hipErrorInvalidValue;
   const dim3 g((unsigned)grid);
   switch (a.group) {

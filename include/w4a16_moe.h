@@ -63,7 +63,9 @@ extern "C" {
 #define W4A16_WS_EXPERT_IDS   1  /* int32 [EM/16]         expert of each block    */
 #define W4A16_WS_HEADER       2  /* int32 [64]: [0] num_tokens_post_padded,
                                     [1] dropped pairs, [2] MFMA tiles,
-                                    [3] GEMV blocks, [4..] reserved              */
+                                    [3] GEMV blocks; with exact-weight tiles
+                                    [2] those and [4], [5] the pair counts
+                                    they may run the GEMV by; the rest reserved  */
 #define W4A16_WS_OFFSETS      3  /* int32 [E+1]           padded expert offsets   */
 #define W4A16_WS_INTER        4  /* bf16  [M*topk, N]     SiLU(gate)*up           */
 #define W4A16_WS_PARTIAL      5  /* bf16  [M*topk, K]     weighted w2 products
