@@ -51,6 +51,7 @@ WS_NFIELDS = 8
 FUSED_BLOCK_M = 16
 GEMV_MAX_TOKENS = 4
 GEMV_ONLY_MAX_M = 24
+EXACT_TILES_MIN_PAIRS = 2
 ALIGN_SCRATCH_MIN_PAIRS = 8192
 
 EXPORTED_SYMBOLS = (

@@ -154,7 +154,8 @@ int small_row_tiles(int64_t n_blocks, int64_t rows) {
 // fragments of a whole group do not fit the registers of taller tiles.
 constexpr int64_t kXTile32MaxPairs = 24;
 constexpr int kXTile128 = 48;
-constexpr int64_t kXTileMinPairs = 2;  // average pairs per expert they start at
+// average pairs per expert they start at
+constexpr int64_t kXTileMinPairs = W4A16_EXACT_TILES_MIN_PAIRS;
 // Row tiles (`rows` outputs each) one workgroup of the exact-weight tiles runs
 // in turn: about 32 steps of 128 elements, so that short reductions do not
 // pay a workgroup's first loads for each row tile, with seven workgroups per CU

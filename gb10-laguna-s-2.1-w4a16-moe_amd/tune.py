@@ -2,8 +2,9 @@
 
 The counterpart of the reference's bench/tune_configs.py, which times Triton
 block-size candidates per M and writes vLLM's per-device config JSON.  Here
-the candidates are the dispatch choices of struct w4a16_moe_tuning (GEMV-only
-vs. GEMV + MFMA split, the split threshold, GEMV token rows per pass); each is
+the candidates are the dispatch choices of struct w4a16_moe_tuning (every
+expert on exact weights vs. GEMV + MFMA split, the split threshold, GEMV token
+rows per pass); each is
 timed on the full-size synthetic layer with HIP-graph replays over rotating
 routing sets (so the weights come from HBM, not the Infinity Cache), under
 both uniform routing and skewed routing (a per-expert logit bias, which gives
@@ -58,12 +59,23 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def effective(M: int, N: int, K: int, t, builtin_tile: int = 192) -> tuple:
-    """What a tuning does at M: the GEMV-only or the split dispatch
-    (builtin_tile: the MFMA tile height mfma_tile_m = 0 selects at M)."""
+def effective(M: int, N: int, K: int, t, builtin_tile: int = 192, layer=None) -> tuple:
+    """What a tuning does at M: the split dispatch, or every expert on exact
+    weights (builtin_tile: the MFMA tile height mfma_tile_m = 0 selects at M).
+    With layer = (topk, E, group), calls on exact weights are told apart as the
+    library runs them: the GEMV routing itself, the GEMV over the sorted
+    blocks, or the exact-weight tiles, which no tuning value changes."""
     if M <= t.gemv_only_max_m or N % 256 or K % 256:
         fused = M <= (t.w2_fused_max_m or 4)
-        return ("gemv", t.gemv_tokens_per_pass, t.gemv_units_per_wg, t.gemv_lanes_per_row,
+        kind = "gemv"
+        if layer is not None:
+            L = _pkg()._lib
+            topk, E, group = layer
+            if L.stage_launches(M, topk, E, N, K, group, t.to_struct())[0] != 0:  # sorts
+                if M * topk >= L.EXACT_TILES_MIN_PAIRS * E:
+                    return ("exact tiles",)
+                kind, fused = "sorted gemv", False
+        return (kind, t.gemv_tokens_per_pass, t.gemv_units_per_wg, t.gemv_lanes_per_row,
                 fused)
     return ("split", t.gemv_max_tokens,
             t.gemv_tokens_per_pass if t.gemv_max_tokens else 0,
@@ -72,10 +84,10 @@ def effective(M: int, N: int, K: int, t, builtin_tile: int = 192) -> tuple:
             t.mfma_tile_m or builtin_tile, t.mfma_row_tiles)
 
 
-def candidates(M: int, N: int, K: int, Tuning, always: int, base=None):
-    """Every distinct dispatch choice worth timing at M, the built-in one
-    (`base`, the library's own choice for M) first; slow candidates are pruned
-    against it."""
+def candidates(M: int, N: int, K: int, Tuning, always: int, base=None, layer=None):
+    """Every distinct dispatch choice worth timing at M (of `layer`, see
+    effective), the built-in one (`base`, the library's own choice for M)
+    first; slow candidates are pruned against it."""
     out = [base if base is not None else Tuning()]
     for tc in (0, 1, 2, 4):
         if tc == 1 and M > 4:
@@ -95,7 +107,7 @@ def candidates(M: int, N: int, K: int, Tuning, always: int, base=None):
     builtin_tile = base.mfma_tile_m if base is not None and base.mfma_tile_m else 192
     seen, uniq = set(), []
     for t in out:
-        key = effective(M, N, K, t, builtin_tile)
+        key = effective(M, N, K, t, builtin_tile, layer)
         if key not in seen:
             seen.add(key)
             uniq.append(t)
@@ -191,7 +203,8 @@ def tune(ms, E, N, K, group, topk, seed=0, check_tol=5e-3):
         base_q = {k: b.quick_us(base) for k, b in benches.items()}
         rows = []
         best = (2.0, base, dict(base_us))
-        for cand in candidates(M, N, K, T.Tuning, T.ALWAYS, base)[1:]:
+        for cand in candidates(M, N, K, T.Tuning, T.ALWAYS, base,
+                               (topk, E, group))[1:]:
             for k, b in benches.items():
                 out = b.call(0, cand).float()
                 torch.cuda.synchronize()

@@ -93,6 +93,11 @@ extern "C" {
  * handful of pairs, and the MFMA launches would only add their fixed cost. */
 #define W4A16_GEMV_ONLY_MAX_M 24
 
+/* Calls that keep every expert on exact weights and do not route themselves
+ * run on MFMA tiles of exact weights from this many pairs per expert (M * topk
+ * / E), on the GEMV over the sorted blocks below. */
+#define W4A16_EXACT_TILES_MIN_PAIRS 2
+
 /*
  * Sizes of moe_align_block_size's outputs.
  * Replaces the buffer sizing of _align_workspace,

@@ -140,6 +140,31 @@ def test_candidates_are_valid(pkg):
         assert any(c.gemv_only_max_m == 0 for c in cands) == (M > 1)
 
 
+@pytest.mark.parametrize("M,N,layer,kinds", [
+    (300, 1408, (6, 64, 128), {"exact tiles"}),        # one dispatch, timed once
+    (25, 1408, (2, 64, 128), {"gemv", "sorted gemv"}),
+    (16, 1024, (10, 256, 32), {"gemv", "split"}),      # routes itself
+    (24, 1024, (16, 64, 32), {"exact tiles", "split"}),  # too many pairs for that
+    (40, 1024, (10, 256, 32), {"sorted gemv", "split"}),
+    (64, 1024, (10, 256, 32), {"exact tiles", "split"})])
+def test_candidates_of_one_dispatch_are_one(pkg, M, N, layer, kinds):
+    """The tuner times each dispatch of a layer once: calls on the exact-weight
+    tiles ignore rows per pass, slabs and lanes per row."""
+    tune = _tune_module(pkg)
+    L = pkg._lib
+    topk, E, group = layer
+    base = pkg.Tuning.from_struct(L.default_tuning(M, topk, E, N, 3072, group))
+    cands = tune.candidates(M, N, 3072, pkg.Tuning, pkg.tuning.ALWAYS, base, layer)
+    keys = [tune.effective(M, N, 3072, t, base.mfma_tile_m, layer) for t in cands]
+    assert len(set(keys)) == len(keys) and {k[0] for k in keys} == kinds
+    assert sum(k[0] == "exact tiles" for k in keys) <= 1
+    # the library lays out a list of tiles for the tiles' calls only
+    for t, k in zip(cands, keys):
+        off = L.workspace_layout_ex(M, topk, E, N, 3072, group, t.to_struct())
+        if k[0] != "split":
+            assert (off[L.WS_GEMV_BLOCKS] - off[L.WS_TILES] > 256) == (k[0] == "exact tiles")
+
+
 # ---------------------------------------------------------------------------
 # GPU
 # ---------------------------------------------------------------------------
