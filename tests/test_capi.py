@@ -301,6 +301,16 @@ def test_workspace_pool_holds_one_buffer_of_the_largest_need(pkg):
     assert pool.cached_bytes() == 0 and pool.retired_bytes() == 0
 
 
+def test_workspace_no_larger_than_the_sorted_blocks(pkg):
+    """Exact-weight tiles: the tile list holds at most one entry per sorted 16-slot block."""
+    L = pkg._lib
+    for M, topk, E in ((30, 10, 256), (50, 10, 256), (777, 6, 64), (2048, 10, 256), (400, 4, 1024)):
+        off = L.workspace_layout(M, topk, E, 128, 1056, 32)
+        _, nb = L.align_sizes(M, topk, E, 16)
+        span = off[L.WS_GEMV_BLOCKS] - off[L.WS_TILES]
+        assert span <= (4 * min(nb, M * topk) + 255) // 256 * 256
+
+
 @pytest.mark.gpu
 def test_capture_id_tells_captures_apart(pkg):
     """0 outside capture; during capture a nonzero id, different for two

@@ -238,11 +238,19 @@ def test_streams_threads_and_growth(pkg, synth, dev):
         x = synth.make_hidden(M, shape.K, dev, seed=M)
         tw, ti = synth.make_routing(M, shape.E, shape.topk, dev, seed=M)
         ins.append((x, *w, tw, ti, 32))
+    pkg.w4a16_moe._WS_POOL.clear()  # stream handles come round again
     want = [pkg.fused_experts_w4a16(*a) for a in ins]
     torch.cuda.synchronize()
-    bad = []
+    bad, done = [], []
 
     def worker():
+        try:
+            calls()
+            done.append(True)
+        except Exception as err:  # (a thread's own ends with it)
+            bad.append(repr(err))
+
+    def calls():
         s = torch.cuda.Stream()
         with torch.cuda.stream(s):
             if pkg._lib.fast().fused(*ins[0]) is not None:
@@ -262,6 +270,7 @@ def test_streams_threads_and_growth(pkg, synth, dev):
     for t in threads:
         t.join()
     assert not bad, bad
+    assert len(done) == len(threads)
 
 
 @pytest.mark.gpu

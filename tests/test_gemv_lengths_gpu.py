@@ -1,6 +1,8 @@
 """GEMV row lengths known only at run time: every remainder of the step ring and
 of the staged pieces, against the oracle, and the one-launch w2 + sum of every
-unrolled length (and past them) against the separate kernels."""
+unrolled length (and past them) against the separate kernels; and the GEMV over
+the sorted blocks, of calls with fewer than two pairs per expert that do not
+route themselves."""
 
 from __future__ import annotations
 
@@ -34,3 +36,28 @@ def test_run_time_lengths(pkg, orc, synth, dev, K, N, M):
     # more) times its ulp: the bound of test_fused_sweep_gpu.py, ~2e-3 of
     # max|out| at a weight of one; few rows, so a flip shows in many of them.
     _check(orc, out, x, w13, w2, s13, s2, tw, ti, 32, tag, mismatch_max=0.05, excess_max=2e-3)
+
+
+@pytest.mark.parametrize("K,N,group", [(1536, 320, 32), (3072, 96, 32), (1024, 448, 64),
+                                       (1280, 384, 128)])
+@pytest.mark.parametrize("M", [25, 47])
+@pytest.mark.parametrize("form", ["uniform", "hot", "dropped"])
+def test_sorted_blocks(pkg, orc, synth, dev, K, N, group, M, form):
+    """hot: one expert in every token (several 16-slot blocks); dropped: ids
+    outside the layer among the others."""
+    tag = f"sorted K={K} N={N} G={group} M={M} {form}"
+    print(tag, flush=True)
+    L = pkg._lib
+    shape = synth.LayerShape(E=128, topk=4, K=K, N=N, group=group)
+    off = L.workspace_layout(M, 4, 128, N, K, group)
+    assert L.stage_launches(M, 4, 128, N, K, group, None) == [1, 1, 1, 1]
+    assert off[L.WS_GEMV_BLOCKS] - off[L.WS_TILES] == 256  # no tiles
+    w13, w2, s13, s2, x, tw, ti = _make(synth, shape, M, dev, seed=K + M)
+    if form == "hot":
+        ti[:, 2] = 7
+    elif form == "dropped":
+        ti[::3, 1] = -1
+        ti[1::3, 3] = 128
+    out = pkg.fused_experts_w4a16(x, w13, w2, s13, s2, tw, ti, group)
+    torch.cuda.synchronize()
+    _check(orc, out, x, w13, w2, s13, s2, tw, ti, group, tag, mismatch_max=0.05, excess_max=2e-3)

@@ -3,8 +3,10 @@ edges of their tiles, row tiles, steps and scale windows.
 
 The calls are the ones that reach them: N or K no multiple of 256, scales that
 are not 16-byte aligned, or a tuning that keeps every expert on exact weights,
-with too many pairs to route themselves and at least two per expert.  No weight is rounded, so
-the bars are the tight ones of test_fused_gpu.py for exact experts.
+with too many pairs to route themselves and at least two per expert; each has
+an expert of more than eight pairs, without which a launch may run the GEMV's
+items.  The header says that tiles were made, and of which height.  No weight
+is rounded, so the bars are the tight ones of test_fused_gpu.py for exact experts.
 """
 
 from __future__ import annotations
@@ -34,6 +36,22 @@ def _case(synth, dev, counts, K, N, group, topk, seed):
     return w13, w2, s13, s2, x, tw, ti
 
 
+# The same below 24 pairs per expert on average: tiles of 32 slots.
+SHORT = [1, 15, 16, 17, 31, 32, 33, 0, 70, 1, 2, 5, 9, 17, 8, 4, 3]
+
+
+def _tiles_ran(pkg, x, ti, w13, w2, group, tile_m, tuning=None):
+    """The last call's launches ran its tiles, of at most tile_m slots each."""
+    L = pkg._lib
+    ws, off = pkg.workspace_tensor(x, ti, w13, w2, group, tuning=tuning)
+    h = ws[off[L.WS_HEADER]: off[L.WS_HEADER] + 24].view(torch.int32).tolist()
+    E = w13.shape[0]
+    flat = ti.reshape(-1).long().cpu()
+    counts = torch.bincount(flat[(flat >= 0) & (flat < E)], minlength=E).tolist()
+    assert h[5] >= 2048, "no expert of more than eight pairs"
+    assert h[2] == sum(-(-c // tile_m) for c in counts)
+
+
 # K, N, group: one 32-element chunk, partial steps and odd step counts, single
 # scales (rows of no whole 16 bytes), scale windows that end inside a row, one
 # row tile and several with an idle tail
@@ -53,11 +71,30 @@ def test_tiles_match_oracle(pkg, orc, synth, dev, K, N, group, counts, topk):
     again = pkg.fused_experts_w4a16(x, w13, w2, s13, s2, tw, ti, group, tuning=t)
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int16), again.view(torch.int16))
+    _tiles_ran(pkg, x, ti, w13, w2, group, 48 if group == 128 else 64, t)
     # A flipped bf16 intermediate moves an output by its weight times the
     # intermediate's ulp: with topk = 1 (weight 1) up to ~2e-3 of max|out|
     # (the bound test_fused_sweep_gpu.py derives per case), at topk = 4 a
     # quarter of that; short reductions (N <= 128 terms) leave max|out| small
     # against one term, hence twice the bound.
+    _check(orc, out, x, w13, w2, s13, s2, tw, ti, group, tag, mismatch_max=0.05,
+           excess_max=4e-3)
+
+
+@pytest.mark.parametrize("K,N,group", SHAPES)
+@pytest.mark.parametrize("topk,dropped", [(1, 0), (4, 100)])
+def test_short_tiles_match_oracle(pkg, orc, synth, dev, K, N, group, topk, dropped):
+    tag = f"short xtile K={K} N={N} G={group} topk={topk} dropped={dropped}"
+    print(tag, flush=True)
+    E = len(SHORT)
+    counts = SHORT + [dropped] if dropped else SHORT
+    assert sum(counts) < 24 * E
+    w13, w2, s13, s2, x, tw, ti = _case(synth, dev, counts, K, N, group, topk, K + N + topk)
+    w13, w2, s13, s2 = (t[:E].contiguous() for t in (w13, w2, s13, s2))
+    t = pkg.Tuning(gemv_only_max_m=pkg.tuning.ALWAYS)
+    out = pkg.fused_experts_w4a16(x, w13, w2, s13, s2, tw, ti, group, tuning=t)
+    torch.cuda.synchronize()
+    _tiles_ran(pkg, x, ti, w13, w2, group, 32, t)
     _check(orc, out, x, w13, w2, s13, s2, tw, ti, group, tag, mismatch_max=0.05,
            excess_max=4e-3)
 
@@ -85,18 +122,9 @@ def test_unaligned_scales_and_fp32_partials(pkg, orc, synth, dev, K, N, group):
     off = pkg.fused_experts_w4a16(x, w13, w2, shifted(s13), shifted(s2), tw, ti, group)
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int16), off.view(torch.int16))
+    _tiles_ran(pkg, x, ti, w13, w2, group, 48 if group == 128 else 64)
     _check(orc, out, x, w13, w2, s13, s2, tw, ti, group, f"unaligned G={group}",
            mismatch_max=0.05)
-
-
-def test_workspace_no_larger_than_the_sorted_blocks(pkg):
-    """The tile list holds at most one entry per sorted 16-slot block."""
-    L = pkg._lib
-    for M, topk, E in ((30, 10, 256), (50, 10, 256), (777, 6, 64), (2048, 10, 256), (400, 4, 1024)):
-        off = L.workspace_layout(M, topk, E, 128, 1056, 32)
-        _, nb = L.align_sizes(M, topk, E, 16)
-        span = off[L.WS_GEMV_BLOCKS] - off[L.WS_TILES]
-        assert span <= (4 * min(nb, M * topk) + 255) // 256 * 256
 
 
 @pytest.mark.parametrize("K,N,group,M", [(1056, 704, 32, 120), (512, 128, 64, 300)])
