@@ -39,7 +39,7 @@ int align_sizes(int64_t M, int64_t topk, int64_t E, int64_t block, int64_t* em,
 
 // Dispatch choices of one call: the public w4a16_moe_tuning, resolved.
 struct Tuning {
-  int gemv_only_max_m;  // M at or below this: every expert on the GEMV kernels
+  int gemv_only_max_m;  // M at or below this: every expert on exact weights
   int gemv_max_tokens;  // above it: experts with more pairs go to MFMA tiles
   int tc;               // GEMV token rows per pass (0 = launcher's choice)
   int tile_m;           // MFMA tile height (0 = built-in, see compute_layout)
@@ -225,8 +225,8 @@ int resolve_tuning(const w4a16_moe_tuning* t, Tuning* out) {
   return W4A16_OK;
 }
 
-// mfma_ok = false keeps every expert on the GEMV kernels (the MFMA kernels
-// read the scales in 16-byte pieces and need them 16-byte aligned).
+// mfma_ok = false keeps every expert on exact weights (the kernels of rounded
+// weights read the scales in 16-byte pieces and need them 16-byte aligned).
 int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
                    int64_t group, const Tuning& T, Layout* L, bool mfma_ok = true) {
   int st = check_gemm_shape(N, K, group);
@@ -257,8 +257,9 @@ int compute_layout(int64_t M, int64_t topk, int64_t E, int64_t N, int64_t K,
   // Below two pairs per expert on average the GEMV over the sorted 16-slot
   // blocks stays: its short work items fill the chip (E=128, top-4, K=1536,
   // N=320: M=25 38.9 against 43.3 us, M=48 50.5 against 57.6, M=64 60.8
-  // against 57.6; E=256, top-10, K=3072, N=128: M=25 60.5 against 64.6, M=39
-  // 80.5 against 70.3).  Under skewed routing the tiles win everywhere (M=25
+  // against 57.6; E=256, top-10, K=3072: N=128 M=25 60.5 against 64.6, M=39
+  // 80.5 against 70.3, N=1056 M=52 316 against 330, M=64 362 against 347: the
+  // line is between them).  Under skewed routing the tiles win everywhere (M=25
   // 57 against 39 us), but the host does not see the routing.  Nor does it see
   // how many pairs belong to experts elsewhere: the tiles' launches look at
   // the sort's counts and run the GEMV's items where few are left
@@ -962,9 +963,9 @@ int w4a16_moe_fused_experts_noalloc(const void* hidden, int64_t ld_hidden,
                                     void* stream, const w4a16_moe_tuning* tuning) {
   // The size check comes first: it needs no device and rejects a call too
   // big for the scratch before anything else runs.  The layout is the one
-  // validate() builds for these pointers (the MFMA kernels need 16-byte
-  // aligned scales; without them every expert runs on the GEMV kernels,
-  // whose work lists are sized differently).
+  // validate() builds for these pointers (the MFMA kernels of rounded weights
+  // need 16-byte aligned scales; without them every expert runs on exact
+  // weights, whose work lists are sized differently).
   Tuning T;
   int st = resolve_tuning(tuning, &T);
   if (st) return st;

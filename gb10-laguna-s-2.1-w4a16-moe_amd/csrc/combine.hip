@@ -7,8 +7,8 @@
 // multiplied by the routing weight) are bf16 like the reference's, or fp32 for
 // calls with M <= 4, the sum is always in slot order from +0.0, and pairs
 // routed to an expert id outside [0, E) -- which the sort skipped, so their
-// partial row was never written -- are left out.  The result is bitwise
-// reproducible.
+// partial row was never written -- are left out (large calls do not load such
+// rows, small ones do and drop them).  The result is bitwise reproducible.
 #include "common.hpp"
 
 namespace w4a16 {
@@ -27,7 +27,8 @@ constexpr int64_t kCombineNtBytes = 2 << 20;
 // One thread owns VPT consecutive outputs of one token (8 for bf16 partials,
 // 4 for fp32: one 16-byte load per slot).  The ids of a batch of slots are
 // read with every slot's partial row (a slot with an id outside [0, E) has an
-// unwritten row: it is read and left out), all in flight together, and the
+// unwritten row: it is read and left out; with NT the ids come first and the
+// row is not read), all in flight together, and the
 // values are added in slot order from +0.0 -- the order of the reference's
 // sum, so the result does not depend on the batching.
 template <bool VEC_STORE, bool BF16, bool NT>

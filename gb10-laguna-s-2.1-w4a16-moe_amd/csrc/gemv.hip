@@ -314,7 +314,9 @@ hipError_t launch_w2_token(const GemvLaunch& a_in, uint16_t* out, int64_t ld_out
   const size_t lds = w2_token_lds_bytes(a.topk, a.kdim);
   // Rows of up to 8 steps (N <= 2048) have all their loads in flight at once;
   // longer ones load a step at a time (E=8, top-2, K=4096, N=1344, M=4
-  // 30.4 -> 24.5 us per call).
+  // 30.4 -> 24.5 us per call; E=64, top-8, K=2048, M=1, with the w13 loop's
+  // change: N=256 7.9 -> 7.6, N=768 12.3 -> 10.2, N=1280 17.5 -> 15.1, N=2048
+  // 27.6 -> 20.7, and past the unrolled ones N=2304 29.7 -> 26.7).
 #define W4A16_W2_TOKEN(NIT)                                                                   \
   case NIT:                                                                                   \
     if (R == 2)                                                                               \

@@ -574,7 +574,9 @@ __device__ __forceinline__ void gemv_item(const GemvLaunch a, int bid, u32x4_t* 
         // Row lengths known only at run time: a piece of every row of the
         // pass per round trip (row by row, each waits for the memory on its
         // own: E=64, top-8, K=2048, N=768, M=12 45.6 -> 40.2 us per call with
-        // the loop of the steps below, which no longer loads past its end).
+        // the loop of the steps below, which no longer loads past its end;
+        // eight shapes from K=1024, N=256 to K=4096, N=2048, M=2-24: 1 to
+        // 17 % less).
         const int n_oct = kdim >> 3;
         const u32x4_t* rows[NTOK];
 #pragma unroll

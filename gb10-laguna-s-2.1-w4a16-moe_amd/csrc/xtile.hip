@@ -35,11 +35,12 @@
 // elements), permuted to the words' code order and stored in fragment order;
 // one barrier per step.
 //
-// Bounds: with many pairs per expert the VALU issue (E=256, K=3072, N=128, 80
-// pairs: w13 80 us, w2 61 us; issue slots busy 86 % of the waves' time on two
-// waves per SIMD, 440 VALU instructions per wave and step of which 192 are
-// the groups' multiply-adds), with few the memory (10 pairs at N=1024: w13
-// 192 us, 4.7 TB/s of weights).
+// Bounds: with many pairs per expert no one unit (E=256, K=3072, N=128, 80
+// pairs: w13 80 us, VALU busy 47 % and MFMA 23 % of the SIMDs' time, 433
+// instructions per wave and step of which 192 are the groups' multiply-adds;
+// w2 61 us, VALU 35 %, its 126 MB of partial rows at 2 TB/s), with 10 the
+// memory (N=1024: w13 192 us, 4.7 TB/s of weights), with few in all the chain
+// of a tile's steps (few_pairs_gemv below).
 #include <limits.h>
 
 #include <algorithm>

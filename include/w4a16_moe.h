@@ -70,11 +70,15 @@ extern "C" {
 #define W4A16_WS_INTER        4  /* bf16  [M*topk, N]     SiLU(gate)*up           */
 #define W4A16_WS_PARTIAL      5  /* bf16  [M*topk, K]     weighted w2 products
                                     (fp32 when M <= 4)                           */
-#define W4A16_WS_TILES        6  /* int32 [tiles][4]      MFMA work list          */
+#define W4A16_WS_TILES        6  /* int32 [tiles][4]      MFMA work list: expert,
+                                    first slot, pairs, 0; exact-weight tiles:
+                                    int32 [tiles], first slot / 16 |
+                                    16-slot blocks << 28                         */
 #define W4A16_WS_GEMV_BLOCKS  7  /* int32 [blocks]        GEMV work list          */
 #define W4A16_WS_NFIELDS      8
-/* Calls with M <= W4A16_GEMV_ONLY_MAX_M skip the align kernel: the GEMV
- * kernels route themselves from topk_ids.  Those calls write only the
+/* Calls with M <= W4A16_GEMV_ONLY_MAX_M and at most 256 pairs (whose routing
+ * fits in LDS) skip the align kernel: the GEMV kernels route themselves from
+ * topk_ids.  Those calls write only the
  * header's dropped count [1], INTER, PARTIAL (not PARTIAL when M <= 4: w2
  * and the top-k sum then run as one kernel) and, in the first M*topk entries
  * of SORTED_IDS, the w13 launch's expert of each work item (-1: none), which
@@ -83,14 +87,15 @@ extern "C" {
 /* Token-block size the fused call uses for its internal expert sort. */
 #define W4A16_FUSED_BLOCK_M 16
 
-/* Experts with more (token, slot) pairs than this run on the MFMA kernels
- * when M > W4A16_GEMV_ONLY_MAX_M and N and K are multiples of 256; the others
- * run on the GEMV kernels. */
+/* Experts with more (token, slot) pairs than this run on the MFMA kernels of
+ * rounded weights when M > W4A16_GEMV_ONLY_MAX_M, N and K are multiples of 256
+ * and the scales 16-byte aligned; the others run on the GEMV kernels. */
 #define W4A16_GEMV_MAX_TOKENS 4
 
-/* Calls with at most this many tokens run every expert on the GEMV kernels
- * (by default; see w4a16_moe_tuning): few experts then hold more than a
- * handful of pairs, and the MFMA launches would only add their fixed cost. */
+/* Calls with at most this many tokens keep every expert on exact weights (by
+ * default; see w4a16_moe_tuning), up to 256 pairs on the GEMV kernels: few
+ * experts then hold more than a handful of pairs, and the MFMA launches would
+ * only add their fixed cost. */
 #define W4A16_GEMV_ONLY_MAX_M 24
 
 /* Calls that keep every expert on exact weights and do not route themselves
