@@ -189,7 +189,7 @@ def load_fast():
     torch."""
     global _fast
     with _lock:
-        if _fast is None:
+        if _fast is None or isinstance(_fast, _NoNativePath):
             if not FAST_PATH.exists():
                 raise ImportError(
                     f"{FAST_PATH} is missing: build it with __graft_entry__.build()")

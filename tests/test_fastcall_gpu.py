@@ -52,6 +52,8 @@ def test_without_the_native_module(pkg, no_native_module, monkeypatch):
              lambda: pkg.moe_align_block_size(t, 16, 4), lambda: pkg.router_topk_softmax(t, 1)]
     with pytest.warns(RuntimeWarning, match="native call path"):
         pkg._lib.fast()
+    with pytest.raises(ImportError):  # (still, with the stand-in in its place)
+        pkg._lib.load_fast()
     for has_library in (True, False):
         if not has_library:
             monkeypatch.setattr(pkg._lib, "LIB_PATH", pkg._lib.FAST_PATH.parent / "none.so")
