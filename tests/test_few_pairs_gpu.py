@@ -15,12 +15,12 @@ pytestmark = pytest.mark.gpu
 OVER = 2048  # header[5] from here on: an expert with more than 8 pairs
 
 
-def _call(synth, dev, counts, E, K, N, group, seed, topk=4):
+def _call(synth, dev, counts, E, K, N, group, seed, topk=4, least=26):
     """Expert e < len(counts) holds counts[e] pairs; dropped pairs (-1 or past
-    the last expert) bring the call to 2 E pairs and past 24 tokens."""
+    the last expert) bring the call to 2 E pairs and `least` tokens."""
     g = torch.Generator().manual_seed(seed)
     live = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))
-    M = max(26, -(-max(2 * E, live.numel()) // topk))
+    M = max(least, -(-max(2 * E, live.numel()) // topk))
     flat = torch.where(torch.rand(M * topk, generator=g) < 0.5, -1, E + 9000)
     flat[: live.numel()] = live
     ti = flat[torch.randperm(M * topk, generator=g)].reshape(M, topk).to(torch.int32).to(dev)
@@ -97,6 +97,23 @@ def test_the_line(pkg, orc, synth, dev, counts, gemv):
     x, w13, w2, s13, s2, tw, ti = args
     _check(orc, out, x, w13, w2, s13, s2, tw, ti, group, f"line {counts[:4]}", mismatch_max=0.05,
            excess_max=4e-3)
+
+
+@pytest.mark.parametrize("counts", [[1, 2, 0, 3, 4, 1, 0, 0], [1, 12, 0, 3, 70, 1, 0, 0]])
+def test_after_the_many_workgroup_sort(pkg, orc, synth, dev, counts):
+    """8,800 pairs, nearly all of them dropped: the sort over many workgroups
+    leaves the same counts."""
+    K, N = 512, 288
+    print(f"few pairs, many workgroups {counts}", flush=True)
+    args = _call(synth, dev, counts, len(counts), K, N, 32, 9, topk=8, least=1100)
+    x, w13, w2, s13, s2, tw, ti = args
+    assert pkg._lib.stage_launches(1100, 8, 8, N, K, 32, None)[0] == 2
+    out, _, header = _run(pkg, args, 32)
+    assert header[4:] == [sum((0, 2, 2, 3, 3)[c] if c < 5 else 6 for c in counts),
+                          sum(OVER if c > 8 else c > 4 for c in counts)]
+    assert header[1] == 8800 - sum(counts) and header[3] == 0
+    _check(orc, out, x, w13, w2, s13, s2, tw, ti, 32, f"many workgroups {counts}",
+           mismatch_max=0.05, excess_max=4e-3)
 
 
 def test_one_share_of_the_experts(pkg, synth, dev):
