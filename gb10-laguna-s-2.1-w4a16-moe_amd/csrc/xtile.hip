@@ -548,12 +548,13 @@ __device__ __forceinline__ void run_xtile(const XtileLaunch& a, int e, int rt0, 
 // w13: while the GEMV is not bound by throughput (few_cost, by what its passes
 // and a tile's steps take: set_few_pairs), or nearly every expert has one or
 // two pairs.  E=32 of 256, K=3072, N=128, 25 and 48 tokens of top-10: w13 27.1
-// -> 10 us, 27.2 -> 18 (the GEMV's own launch 9.8 and 17.0).
+// -> 10 us, 27.2 -> 18 (the GEMV's own launch 9.8 and 17.0); the calls 44.5 ->
+// 30.6 and 45.0 -> 36.7.
 // w2: while no expert takes a second pass (N=1056, K=3072: 20 experts of 1, 4
 // and 8 pairs 13, 17 and 29 us against 28 to 29; 240 of them 123, 151 and 297
 // against 154 to 164) and, for short rows, whose tiles are short too, the
-// items are few.  The branch costs the launches that run their tiles 0 to 0.4
-// us, those of 16-slot tiles with groups of 64 (other registers) 0.7 to 1.
+// items are few.  The branch costs the launches that run their tiles 0 to 0.3
+// us, those of 16-slot tiles with groups of 64 (other registers) 0.3 to 0.7.
 template <int MODE>
 __device__ __forceinline__ bool few_pairs_gemv(const XtileLaunch& a, int experts, int cost,
                                                int over) {
@@ -570,32 +571,44 @@ __host__ __device__ constexpr int gemv_groups(int mode, int n_out) {
   return (n_out + 8 * gemv_rpl(mode) * kWaves - 1) / (8 * gemv_rpl(mode) * kWaves);
 }
 
+// A function of its own, which gets the launch's arguments by their address
+// and the workgroup's LDS by its offset, both uniform: inlined, it took scalar
+// registers from the tiles (w2 of 64-slot tiles spilled 64, now 21) and a call
+// of 2,048 tokens at N=128 1 us; the call costs the GEMV's launches 0.4 us.
 template <int MODE, int TC>
-__device__ __forceinline__ void run_gemv(const XtileLaunch& a, int experts, unsigned char* lds) {
+__device__ __attribute__((noinline)) void run_gemv(uint32_t args_lo, uint32_t args_hi,
+                                                   uint32_t lds_at, int first, int stride,
+                                                   int experts) {
   static_assert(gemv_dev::kGemvWaves == kWaves, "workgroups of one size");
+  auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+  const auto* a = (const __attribute__((address_space(4))) XtileLaunch*)(
+      (uint64_t)uniform(args_lo) | (uint64_t)uniform(args_hi) << 32);
+  auto* lds =
+      (gemv_dev::u32x4_t*)(__attribute__((address_space(3))) gemv_dev::u32x4_t*)uniform(lds_at);
   GemvLaunch g{};
-  g.act = a.act;
-  g.ld_act = a.ld_act;
-  g.w = a.w;
-  g.s = a.s;
-  g.sorted = a.sorted;
-  g.expert_ids = a.expert_ids;
-  g.header = a.header;
-  g.topk_w = a.topk_w;
-  g.out = a.out;
-  g.partial_bf16 = a.partial_bf16;
-  g.n_tok = a.n_tok;
-  g.topk = a.topk;
-  g.n_out = a.n_out;
-  g.kdim = a.kdim;
+  g.act = a->act;
+  g.ld_act = a->ld_act;
+  g.w = a->w;
+  g.s = a->s;
+  g.sorted = a->sorted;
+  g.expert_ids = a->expert_ids;
+  g.header = a->header;
+  g.topk_w = a->topk_w;
+  g.out = a->out;
+  g.partial_bf16 = a->partial_bf16;
+  g.n_tok = a->n_tok;
+  g.topk = a->topk;
+  g.n_out = a->n_out;
+  g.kdim = a->kdim;
   g.block = 16;
-  g.group = a.group;
-  g.nib_mask = a.nib_mask;
-  g.nib_magic = a.nib_magic;
-  const int items = experts * gemv_groups(MODE, a.n_out);
-  for (int i = (int)blockIdx.x; i < items; i += (int)gridDim.x)
-    gemv_dev::gemv_item<MODE, gemv_rpl(MODE), gemv_pf(MODE), TC, kWaves, 0, false, 1, 8>(
-        g, i, reinterpret_cast<gemv_dev::u32x4_t*>(lds));
+  g.group = a->group;
+  g.nib_mask = a->nib_mask;
+  g.nib_magic = a->nib_magic;
+  const int items = (int)uniform(experts) * gemv_groups(MODE, g.n_out);
+  const int step = (int)uniform(stride);
+  for (int i = (int)uniform(first); i < items; i += step)
+    gemv_dev::gemv_item<MODE, gemv_rpl(MODE), gemv_pf(MODE), TC, kWaves, 0, false, 1, 8>(g, i,
+                                                                                         lds);
 }
 
 template <int MODE, int GS, int SP, class X>
@@ -616,10 +629,14 @@ void xtile_kernel(const XtileLaunch a) {
   const int tile = kXcds * round + ((round & 1) ? kXcds - 1 - xcd : xcd);
   const int experts = a.header[0] >> 4;
   if (few_pairs_gemv<MODE>(a, experts, a.header[4], a.header[5])) {
+    const uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();  // = &a
+    const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds;
     if (MODE == 1 || gemv_dev::gemv_lds_bytes(4, a.kdim) <= kGemvLds)
-      run_gemv<MODE, 4>(a, experts, lds);
+      run_gemv<MODE, 4>((uint32_t)args, (uint32_t)(args >> 32), at, (int)blockIdx.x,
+                        (int)gridDim.x, experts);
     else
-      run_gemv<MODE, MODE == 0 ? 2 : 4>(a, experts, lds);
+      run_gemv<MODE, MODE == 0 ? 2 : 4>((uint32_t)args, (uint32_t)(args >> 32), at,
+                                        (int)blockIdx.x, (int)gridDim.x, experts);
     return;
   }
   if (tile >= a.header[2]) return;
